@@ -43,19 +43,21 @@ def _two_sided(X: Tensor, left: Tensor, right: Tensor) -> Tensor:
 
 
 def _two_sided_inverse(X: Tensor, left: Tensor, right: Tensor) -> Tensor:
-    """(T_m X T_n) (.) left[:, None] (.) right[None, :] (quipsharp/incoherence.py:74-83)."""
-    _lib.require_gpu(X, what="incoherence processing")
+    """(T_m X T_n) (.) left[:, None] (.) right[None, :] (quipsharp/incoherence.py:74-83).
+    The row signs are applied before T_n, which they pass through unchanged."""
+    _lib.require_gpu(X, left, right, what="incoherence processing")
     X = X.float().contiguous()
     m, n = X.shape
+    left, right = left.float().expand(m).contiguous(), right.float().expand(n).contiguous()
     fm, fn = kron_factor(m), kron_factor(n)
     Km = hartley_matrix(fm[0], X.device) if fm[0] > 1 else None
     Kn = hartley_matrix(fn[0], X.device) if fn[0] > 1 else None
     L = _lib.lib()
     s = _lib.stream_of(X)
     out = torch.empty_like(X)
-    _lib.check(L.qs_rht_f32(_lib.ptr(X), _lib.ptr(out), 1, m, n, None, None, None, fm[0], _lib.ptr(Km), s))
-    _lib.check(L.qs_rht_f32(_lib.ptr(out), _lib.ptr(out), m, n, 1, None, None, None, fn[0], _lib.ptr(Kn), s))
-    return out * left.unsqueeze(1) * right.unsqueeze(0)
+    _lib.check(L.qs_rht_f32(_lib.ptr(X), _lib.ptr(out), 1, m, n, None, None, _lib.ptr(left), fm[0], _lib.ptr(Km), s))
+    _lib.check(L.qs_rht_f32(_lib.ptr(out), _lib.ptr(out), m, n, 1, None, None, _lib.ptr(right), fn[0], _lib.ptr(Kn), s))
+    return out
 
 
 def _rows(x: Tensor, pre: Tensor = None, post: Tensor = None) -> Tensor:
