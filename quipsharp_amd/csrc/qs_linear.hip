@@ -697,7 +697,9 @@ static int forward_wide(const void* x, int x_dtype, int64_t ldx, int64_t batch, 
   P.sbits = sbits;
   int rc = QS_OK;
   const bool sv_aligned = (reinterpret_cast<uintptr_t>(sv) & (sbits ? 3 : 15)) == 0;
-  if (chunk_transform_fits(n, kron_pn) && sv_aligned)
+  if (rows_input_fits(P))
+    rc = launch_wx(&P, 1, s);
+  else if (chunk_transform_fits(n, kron_pn) && sv_aligned)
     rc = launch_bx_rows(P, s);
   else if (big_input_fits(n, kron_pn, x_dtype) && sv_aligned && fused_x_aligned(x, x_dtype, ldx))
     rc = launch_bx_big(P, s);
@@ -724,6 +726,7 @@ static int forward_wide(const void* x, int x_dtype, int64_t ldx, int64_t batch, 
   if (mv_end) QS_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(mv_end), s));
   // partial groups summed by the output kernels; the +-1/4 shifts are in y1
   P.SG = F.SGk;
+  if (rows_output_fits(P)) return launch_wy(&P, 1, s);
   if (chunk_transform_fits(m, kron_pm)) return launch_by_rows(P, s);
   if (big_transform_fits(m, kron_pm)) return launch_by_big(&P, 1, s);
   return launch_yout_rows(P.y1p, F.SGk, (int)batch, m, kron_pm, kron_m, nullptr, 0, P.xmul, s0, layer_scale, su, bias,
@@ -1123,7 +1126,9 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
     }
     off += W.total;
   }
-  int rc = launch_bx_group(P, count, s, pre);
+  bool rows_in = wide && !pre;
+  for (int g = 0; g < count; ++g) rows_in = rows_in && rows_input_fits(P[g]);
+  int rc = rows_in ? launch_wx(P, count, s) : launch_bx_group(P, count, s, pre);
   if (rc) return rc;
   if (wide) {
     if (mv_begin) QS_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(mv_begin), s));
@@ -1166,9 +1171,13 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
   }
   // output transforms: the chunk-scheme ones in one launch, those up to
   // 32768 in another, the others one by one
-  BatchedPass Pc[QS_MAX_GROUP], Pb[QS_MAX_GROUP];
-  int nc = 0, nb = 0;
+  BatchedPass Pc[QS_MAX_GROUP], Pb[QS_MAX_GROUP], Pr[QS_MAX_GROUP];
+  int nc = 0, nb = 0, nr = 0;
   for (int g = 0; g < count; ++g) {
+    if (wide && rows_output_fits(P[g])) {
+      Pr[nr++] = P[g];
+      continue;
+    }
     if (chunk_transform_fits(P[g].m, P[g].pm)) {
       Pc[nc++] = P[g];
       continue;
@@ -1179,6 +1188,10 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
     }
     rc = launch_yout_rows(P[g].y1p, P[g].SG, (int)batch, P[g].m, P[g].pm, P[g].Km, nullptr, 0, P[g].xmul, P[g].s0,
                           P[g].layer_scale, P[g].su, P[g].bias, P[g].y, y_dtype, P[g].ldy, s);
+    if (rc) return rc;
+  }
+  if (nr) {
+    rc = launch_wy(Pr, nr, s);
     if (rc) return rc;
   }
   if (nb) {

@@ -126,6 +126,16 @@ bool big_input_fits(int64_t n, int p, int x_dtype);
 int launch_bx_big(const BatchedPass& P, hipStream_t stream);
 int launch_by_big(const BatchedPass* P, int count, hipStream_t stream);
 
+// Transforms of a long batch (qs_linear_rows.hip), one row per wave: the input
+// side from kRowsInMin rows and for every length on the chunk scheme up to 32768
+// (each row and its signs on 16 bytes), the output side from kRowsOutMin rows
+// for lengths beyond the chunk kernels' 12288.
+constexpr int64_t kRowsInMin = 160, kRowsOutMin = 320;
+bool rows_input_fits(const BatchedPass& P);
+bool rows_output_fits(const BatchedPass& P);
+int launch_wx(const BatchedPass* P, int count, hipStream_t stream);
+int launch_wy(const BatchedPass* P, int count, hipStream_t stream);
+
 // Fragment-major fp16 operand of the wide GEMM: row b, columns k .. k + 7 (k
 // a multiple of 8) are one 16-byte word, words ordered by [b / 16][k / 256]
 // [(k / 8) % 8][(k % 256) / 64][b % 16], so that the 64 lanes of a wave read
