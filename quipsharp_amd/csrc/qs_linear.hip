@@ -721,7 +721,7 @@ static int forward_wide(const void* x, int x_dtype, int64_t ldx, int64_t batch, 
   F.sgf = P.sg;
   F.y1p = P.y1p;
   F.SGk = wide_splits(m, n, batch, cu_count(), codes1 != nullptr);
-  rc = launch_linear_wide_mfma(F, s);
+  rc = launch_linear_wide(&F, 1, s);
   if (rc) return rc;
   if (mv_end) QS_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(mv_end), s));
   // partial groups summed by the output kernels; the +-1/4 shifts are in y1
@@ -1070,8 +1070,8 @@ size_t group_prefix_bytes(int count, int64_t n, M m_of) {
 
 // Grouped forward for three or more rows: the input transforms of all the
 // linears in one launch, their decode-matvecs in one launch (16-row pass) or
-// one wide GEMM each (kWideMinBatch rows and more; above 128 rows one GEMM
-// for linears of one shape whose tiles fit one round over the CUs), and their
+// one wide GEMM (kWideMinBatch rows and more; beyond 128 rows of one stage one
+// each, or one for linears of one shape whose tiles fit one round over the CUs), and their
 // output transforms in one launch (a linear whose m is outside the chunk
 // scheme: the whole-row output kernel).  Bit-identical to one
 // qs_linear_forward per linear, except a shared GEMM: its slice groups are the
@@ -1137,6 +1137,10 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
     bool one_shape = true;
     for (int g = 0; g < count; ++g) one_shape = one_shape && P[g].m == P[0].m && P[g].codes1 == nullptr;
     const int gsk = one_shape ? wide_group_splits(P[0].m, n, batch, count, cu_count()) : 0;
+    bool shared = true;
+    for (int g = 0; g < count; ++g)
+      shared = shared && (P[g].codes1 != nullptr) == (P[0].codes1 != nullptr) &&
+               wide_shares_launch(batch, P[g].codes1 != nullptr);
     WideMfma F[QS_MAX_GROUP];
     for (int g = 0; g < count; ++g) {
       F[g] = WideMfma{};
@@ -1151,14 +1155,14 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
       F[g].sgf = P[g].sg;
       F[g].y1p = P[g].y1p;
       F[g].SGk = gsk ? gsk : wide_splits(P[g].m, n, batch, cu_count(), P[g].codes1 != nullptr);
-      if (!gsk) {
-        rc = launch_linear_wide_mfma(F[g], s);
+      if (!gsk && !shared) {
+        rc = launch_linear_wide(&F[g], 1, s);
         if (rc) return rc;
       }
       P[g].SG = F[g].SGk;  // partial groups summed by the output kernels
     }
-    if (gsk) {
-      rc = launch_linear_wide_group(F, count, s);
+    if (gsk || shared) {
+      rc = launch_linear_wide(F, count, s);
       if (rc) return rc;
     }
     if (mv_end) QS_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(mv_end), s));

@@ -176,17 +176,21 @@ struct WideMfma {
 // round over the CUs (a partial second round costs more than the split
 // saves: 11008 x 4096 at 512 rows, 172 tiles, runs 3.7 % faster over the
 // step as 1 group than as 2), at most the output kernel's partial-group
-// limit.
+// limit.  Up to 128 rows two work-groups per CU, which run side by side and
+// cover each other's loads, while the partial sums take at most 8 MiB.
 int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2);
 // Linears of one shape (m, n, B) with one stage above 128 rows whose tiles
 // together fit one round over the CUs share one producer / consumer GEMM
-// launch (launch_linear_wide_group), with the slice groups chosen for the
+// launch (launch_linear_wide), with the slice groups chosen for the
 // whole group (fewer than each would take alone, so their outputs equal
 // separate calls up to the fp32 summation order).  Returns those slice
 // groups, or 0 when the linears take one launch each.
 int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu);
-int launch_linear_wide_group(const WideMfma* G, int count, hipStream_t stream);
-int launch_linear_wide_mfma(const WideMfma& G, hipStream_t stream);
+// Whether linears of B rows of one operand width share a launch whatever their
+// m, each with its own slice groups (the decode-in-the-loop kernel), or only
+// those of one shape by wide_group_splits (the producer / consumer kernel).
+bool wide_shares_launch(int64_t B, bool has2);
+int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream);
 
 
 }  // namespace qs

@@ -26,181 +26,167 @@ constexpr int kDqOffLut1 = 32768;          // 256 x uint4 (E8 1-bit rows, fp16)
 // ---------------------------------------------------------------------------
 // Decode in the GEMM loop
 // ---------------------------------------------------------------------------
-// Work-group: 4 waves, 128 weight rows (8 code tiles of 16 rows) x 128
-// activation rows; wave w multiplies all 128 weight rows by activation rows
-// 32 w .. 32 w + 31 (two 16-row MFMA column tiles), so every decoded A
-// fragment feeds two MFMAs (four with a second stage) and every B fragment
-// (1 KiB, one coalesced load from the fragment-major operand) eight.  The
-// code tiles of a slice are copied into LDS once per work-group (double
-// buffered, one barrier per slice); every wave decodes all of them itself
-// (VALU work that overlaps the matrix cores) rather than sharing decoded
-// fragments through LDS.
+// A work-group's 4 waves take 128 weight rows and up to 128 activation rows.
+// Two reads bound the loop: the LDS tables (two words a code, 16 bytes more with
+// a second stage: 10 and 26 clocks per 64 codes) and the operand through the
+// L1 (1 KiB a fragment, 16 clocks).  With WC = 1 every wave has two 16-row code
+// tiles of its own and multiplies all of the activation rows, so that a code is
+// decoded once and a fragment read four times; with WC = 2, beyond 64 rows of
+// one stage, the waves are 2 x 2, four code tiles by half the rows each, both
+// twice.  (A wave with all the weight rows and activation rows of its own, as
+// this kernel was, decodes every code four times.)  A wave's code tiles go from
+// memory to its registers a slice ahead, and the loop has no barrier.
+//
+// A layer's linears and transforms, graph-replayed (that form -> now):
+//   Llama-3-8B 3 bits  17 rows 178 -> 127 us, 45 202 -> 163, 128 308 -> 267, 700 1256 -> 1154
+//   Qwen3-32B 2 bits   17 rows 250 -> 184 us, 45 291 -> 239, 64 325 -> 272
+//   the same, 128 rows 437 -> 417 us (WC = 1: 520); 3 bits 559 -> 501 (WC = 2: 522)
+//
+// Linears of one operand width share a launch, each with the slice groups that
+// it has alone, so that the outputs do not depend on the company.
 constexpr int kWgThreads = 256;
-constexpr int kWgRowTiles = 8;     // 16-row code tiles per work-group
 constexpr int kWgWaves = kWgThreads / 64;
-// 16-row activation tiles per wave (CT): four (64 activation rows per wave,
-// 256 per work-group) for wide batches, two with a second stage (whose
-// accumulators take the registers), and fewer for short batches so that no
-// wave multiplies tiles past the last row.  Wave w of work-group column ct
-// takes tiles 4 CT ct + w + 4 t, t < CT.
-inline int wg_ct(int64_t B, bool has2) {
-  const int64_t nbt = (B + 15) / 16;
-  const int ct = nbt <= kWgWaves ? 1 : nbt <= 2 * kWgWaves ? 2 : 4;
-  return has2 && ct > 2 ? 2 : ct;
-}
-constexpr int kWgRows = 16 * kWgRowTiles;
-constexpr int kWgCodeBuf = kWgRowTiles * 1024;           // code bytes of one slice
-constexpr int kWgOffCodes = kDqOffLut1 + 4096;           // 2 slices
-constexpr int kWgOffCodes1 = kWgOffCodes + 2 * kWgCodeBuf;  // 2 slices of second-stage bytes
-constexpr int kWgLds = kWgOffCodes1 + kWgCodeBuf;
-constexpr int kWgRing = 4;         // B fragments in flight per wave (steps of 32 columns)
-constexpr int kWgAhead = 3;        // steps between a B load and its use
-static_assert(kWgLds <= 65536, "LDS budget");
-constexpr int kWgCopies = kWgCodeBuf / (16 * kWgThreads);  // 16-byte code copies per thread and slice
-static_assert(kWgCopies >= 1 && kWgCopies <= 2 && kWgCopies * 16 * kWgThreads == kWgCodeBuf, "code copy");
+constexpr int kWgRowTiles = 8;                       // 16-row code tiles of a work-group
+constexpr int kWgMaxCols = 8;                        // 16-row activation tiles of a work-group
+constexpr int kWgLds = kDqOffLut1 + 4096;
+constexpr int64_t kWgPartialBytes = 8 << 20;         // of partial sums for a second work-group per CU
 static_assert(kWgThreads >= 256, "E8 one-bit table rows: one per thread of the first 256");
 
-// One linear of a wp_kernel launch: linears of one shape (m, n, rows) that
-// read their own operands share a launch, job j taking tiles j T1 .. (j + 1)
-// T1 - 1 of the grid's tile order (T1 = nrt nct SGk).
+// Activation tiles per work-group: the tiles dealt evenly over as few
+// work-group columns as take them, rounded up to a compiled width.
+inline int wg_cols(int64_t B) {
+  const int64_t nbt = (B + 15) / 16, nct = (nbt + kWgMaxCols - 1) / kWgMaxCols;
+  const int64_t nb = (nbt + nct - 1) / nct;
+  return nb <= 2 ? 2 : nb <= 3 ? 3 : nb <= 4 ? 4 : nb <= 6 ? 6 : 8;
+}
+// Single-stage calls of more than 128 rows run wp_kernel (256 activation rows
+// per work-group).
+inline bool use_wp(int64_t B, bool has2) { return !has2 && B > 16 * kWgMaxCols; }
+
+// One linear of a launch.  wp_kernel: linears of one shape (m, n, rows) that
+// read their own operands share a launch, job j taking tiles j T1 .. (j + 1) T1
+// - 1 of the grid's tile order (T1 = nrt nct SGk).
 struct WpJob {
   const uint16_t* codes0;
   const _Float16* x2f;
   float* y1p;
   float s0;
+  // wg_kernel
+  const uint8_t* codes1;
+  const _Float16* sgf;
+  float s1;
+  int m, RB, nrt, SGk, spg;
+  int t0;              // first tile of the launch
 };
 
 struct WgArgs {
-  const uint16_t* codes0;
-  const uint8_t* codes1;
-  const _Float16* x2f;
-  const _Float16* sgf;
-  float* y1p;
   int m, B, S, RB;     // RB: 16-row blocks
   int nrt, nct;        // work-group tiles along the weight rows / activation rows
   int SGk, spg;        // slice groups, slices per group
-  float s0, s1;
-  int njobs;           // wp_kernel: linears of the launch (job[0]: the fields above)
+  int njobs;
+  int tiles;           // wg_kernel: of all jobs
   WpJob job[QS_MAX_GROUP];
 };
 
-template <bool HAS2, int kWgColTiles>
-__global__ __launch_bounds__(kWgThreads) void wg_kernel(WgArgs A) {
+template <bool HAS2, int NB, int WC>
+__global__ __launch_bounds__(kWgThreads, 2) void wg_kernel(WgArgs A) {
+  constexpr int RT = kWgRowTiles * WC / kWgWaves;  // code tiles of a wave
+  // steps between an operand load and its use (one where two stages' sums take the registers)
+  constexpr int kAhead = NB <= 4 ? 3 : 1, kRing = kAhead + 1;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   uint4* lut1 = reinterpret_cast<uint4*>(lds + kDqOffLut1);
   const int tid = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane >> 4, r16 = lane & 15;
 
   // Tiles are ordered weight-row tiles fastest, then activation tiles, then
-  // slice groups, and dealt to the XCDs in contiguous runs: work-group i runs
-  // on XCD i % 8, so tile (i % 8) * ceil(T / 8) + i / 8 keeps each XCD's L2 on
-  // a few activation columns and slice groups (the grid is rounded up to a
-  // multiple of 8; the surplus work-groups exit at once).
-  const int T = A.nrt * A.nct * A.SGk;
-  const int per = (T + 7) >> 3;
+  // slice groups, then jobs, and dealt to the XCDs in contiguous runs:
+  // work-group i runs on XCD i % 8, so tile (i % 8) * ceil(T / 8) + i / 8 keeps
+  // each XCD's L2 on a few activation columns and slice groups (the grid is
+  // rounded up to a multiple of 8; the surplus work-groups exit at once).
+  const int per = (A.tiles + 7) >> 3;
   int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-  if (bid >= T) return;
-  const int rt = bid % A.nrt;
-  bid /= A.nrt;
+  if (bid >= A.tiles) return;
+  int jj = 0;
+#pragma unroll
+  for (int k = 1; k < QS_MAX_GROUP; ++k)
+    if (k < A.njobs && bid >= A.job[k].t0) jj = k;
+  const WpJob& J = A.job[jj];
+  bid -= J.t0;
+  const int rt = bid % J.nrt;
+  bid /= J.nrt;
   const int ct = bid % A.nct;
   const int g = bid / A.nct;
-  const int s_begin = g * A.spg;
-  const int s_end = s_begin + A.spg < A.S ? s_begin + A.spg : A.S;
+  const int s_begin = g * J.spg;
+  const int s_end = s_begin + J.spg < A.S ? s_begin + J.spg : A.S;
   const int s_last = s_end > s_begin ? s_end - 1 : (A.S - 1);  // an empty group reads, never uses, slice S - 1
 
-  // Global bytes of a slice's code tiles: thread tid copies bytes 16 tid
-  // (and 16 tid + 16 kWgThreads) of the 8 KiB (tile = byte / 1024), threads
-  // below 256 byte 16 tid of the 4 KiB second stage (tile = byte / 512).  Row
-  // blocks past the end read the last one (decoded, never stored).
-  auto tile_of = [&](int i, int s) -> size_t {
-    int rb = rt * kWgRowTiles + i;
-    rb = rb < A.RB ? rb : A.RB - 1;
+  // this wave's code tiles; row blocks past the end read the last one (decoded, never stored)
+  const int rb0 = rt * kWgRowTiles + w / WC * RT;
+  uint4 cw[RT], nw[RT];
+  uint2 cw1[RT], nw1[RT];
+  auto load_codes = [&](int s) __attribute__((always_inline)) {
     s = s < s_last ? s : s_last;
-    return (size_t)rb * A.S + s;
-  };
-  struct CodeCopy {
-    uint4 c0, c1, c2;  // bytes 16 tid, 16 (tid + kWgThreads) of the codes; 16 tid of the second stage
-  };
-  auto load_codes = [&](int s) -> CodeCopy {
-    CodeCopy r;
-    const int b0 = 16 * tid, b1 = 16 * (tid + kWgThreads);
-    const char* c0 = reinterpret_cast<const char*>(A.codes0);
-    r.c0 = ld_nt_u4(c0 + tile_of(b0 >> 10, s) * 1024 + (b0 & 1023));
-    r.c1 = kWgCopies > 1 ? ld_nt_u4(c0 + tile_of(b1 >> 10, s) * 1024 + (b1 & 1023)) : make_uint4(0, 0, 0, 0);
-    r.c2 = HAS2 && tid < 256 ? ld_nt_u4(A.codes1 + tile_of(b0 >> 9, s) * 512 + (b0 & 511)) : make_uint4(0, 0, 0, 0);
-    return r;
-  };
-  auto store_codes = [&](int p, const CodeCopy& r) {
-    *reinterpret_cast<uint4*>(lds + kWgOffCodes + p * kWgCodeBuf + 16 * tid) = r.c0;
-    if (kWgCopies > 1) *reinterpret_cast<uint4*>(lds + kWgOffCodes + p * kWgCodeBuf + 16 * (tid + kWgThreads)) = r.c1;
-    if (HAS2 && tid < 256) *reinterpret_cast<uint4*>(lds + kWgOffCodes1 + p * (kWgCodeBuf / 2) + 16 * tid) = r.c2;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const int rb = rb0 + i < J.RB ? rb0 + i : J.RB - 1;
+      const size_t tile = (size_t)rb * A.S + s;
+      nw[i] = ld_nt_u4(reinterpret_cast<const char*>(J.codes0) + tile * 1024 + 16 * lane);
+      if (HAS2) nw1[i] = *reinterpret_cast<const uint2*>(J.codes1 + tile * 512 + 8 * lane);
+    }
   };
 
-  // activation tiles of this wave (clamped to the last one: computed, never stored)
+  // activation tiles (clamped to the last one: computed, never stored)
   const int nbt = (A.B + 15) >> 4;
-  const _Float16* xb[kWgColTiles];
-  const _Float16* sb[kWgColTiles];
+  const _Float16* xb[NB];
+  const _Float16* sb[NB];
 #pragma unroll
-  for (int t = 0; t < kWgColTiles; ++t) {
-    int c = kWgWaves * kWgColTiles * ct + w + kWgWaves * t;
+  for (int t = 0; t < NB; ++t) {
+    int c = NB * (WC * ct + w % WC) + t;
     c = c < nbt ? c : nbt - 1;
-    xb[t] = A.x2f + (size_t)c * A.S * 8 * 512 + 8 * lane;  // + (s * 8 + step) * 512 halves
-    sb[t] = A.sgf + (size_t)c * A.S * 512 + 8 * lane;      // + s * 512 halves
+    xb[t] = J.x2f + (size_t)c * A.S * 8 * 512 + 8 * lane;  // + (s * 8 + step) * 512 halves
+    sb[t] = J.sgf + (size_t)c * A.S * 512 + 8 * lane;      // + s * 512 halves
   }
-  half8 bring[kWgRing][kWgColTiles];
-  auto load_b = [&](int s, int step, half8 (&dst)[kWgColTiles]) {
+  half8 bring[kRing][NB];
+  auto load_b = [&](int s, int step, half8 (&dst)[NB]) __attribute__((always_inline)) {
     s = s < s_last ? s : s_last;
 #pragma unroll
-    for (int t = 0; t < kWgColTiles; ++t)
-      dst[t] = *reinterpret_cast<const half8*>(xb[t] + ((size_t)s * 8 + step) * 512);
+    for (int t = 0; t < NB; ++t) dst[t] = *reinterpret_cast<const half8*>(xb[t] + ((size_t)s * 8 + step) * 512);
   };
 
-  // a wave with no activation tile of its own only helps copy the codes
-  // (with four tiles per wave, chosen for long batches, every wave but those
-  // of a ragged last column has work: no branch)
-  const bool wave_on = kWgColTiles == 4 || kWgWaves * kWgColTiles * ct + w < nbt;
-  CodeCopy gc = load_codes(s_begin);
-  if (wave_on) {
+  load_codes(s_begin);
 #pragma unroll
-    for (int k = 0; k < kWgAhead; ++k) load_b(s_begin, k, bring[k]);
-  }
+  for (int k = 0; k < kAhead; ++k) load_b(s_begin, k, bring[k]);
   {
     LutCopy<kWgThreads> lc;
     load_luts(tid, lc);
     uint4 t1 = make_uint4(0, 0, 0, 0);
-    if (HAS2 && tid < 256) t1 = *reinterpret_cast<const uint4*>(kE81h.w[tid]);
+    if (HAS2) t1 = *reinterpret_cast<const uint4*>(kE81h.w[tid]);
     store_luts(lds, tid, lc);
-    if (HAS2 && tid < 256) lut1[tid] = t1;
+    if (HAS2) lut1[tid] = t1;
   }
-  store_codes(0, gc);
-  __syncthreads();  // LUTs and the first slice's code tiles complete
+  __syncthreads();  // LUTs complete
 
-  floatx4 acc[kWgRowTiles][kWgColTiles];
-  floatx4 acc2[kWgRowTiles][kWgColTiles];
+  floatx4 acc[RT][NB];
+  floatx4 acc2[RT][NB];
 #pragma unroll
-  for (int i = 0; i < kWgRowTiles; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int t = 0; t < kWgColTiles; ++t) {
+    for (int t = 0; t < NB; ++t) {
       acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
       acc2[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
   for (int s = s_begin; s < s_end; ++s) {
-    const int p = (s - s_begin) & 1;
-    uint4 cw[kWgRowTiles];
-    uint2 cw1[kWgRowTiles];
 #pragma unroll
-    for (int i = 0; i < kWgRowTiles; ++i) {
-      cw[i] = *reinterpret_cast<const uint4*>(lds + kWgOffCodes + p * kWgCodeBuf + 1024 * i + 16 * lane);
-      if (HAS2)
-        cw1[i] = *reinterpret_cast<const uint2*>(lds + kWgOffCodes1 + p * (kWgCodeBuf / 2) + 512 * i + 8 * lane);
+    for (int i = 0; i < RT; ++i) {
+      cw[i] = nw[i];
+      if (HAS2) cw1[i] = nw1[i];
     }
-    gc = load_codes(s + 1);  // the next slice's tiles, stored after this slice
-    if (wave_on) {
-    half8 sgs[kWgColTiles];  // group sums / 4 of this slice, used after its 8 steps
+    load_codes(s + 1);
+    half8 sgs[NB];  // group sums / 4 of this slice, used after its 8 steps
 #pragma unroll
-    for (int t = 0; t < kWgColTiles; ++t) sgs[t] = *reinterpret_cast<const half8*>(sb[t] + (size_t)s * 512);
+    for (int t = 0; t < NB; ++t) sgs[t] = *reinterpret_cast<const half8*>(sb[t] + (size_t)s * 512);
 
     auto word = [&](int i, int c) -> uint32_t {
       return c < 2 ? cw[i].x : c < 4 ? cw[i].y : c < 6 ? cw[i].z : cw[i].w;
@@ -208,16 +194,12 @@ __global__ __launch_bounds__(kWgThreads) void wg_kernel(WgArgs A) {
     // LUT words of step c + 1 are read while the MFMAs of step c run, and the
     // fp16 A fragments of step c + 1 are built between them, so neither the
     // LDS latency nor the decode VALU work stalls the matrix cores.
-    uint32_t hv[kWgRowTiles], lv[kWgRowTiles];
-    half8 l1[2][kWgRowTiles];
-    auto read_luts = [&](int c) {
+    uint32_t hv[RT], lv[RT];
+    half8 l1[2][RT];
+    auto read_luts = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < kWgRowTiles; ++i) {
-        const uint32_t v = word(i, c);
-        const uint32_t ha = (c & 1) ? ((v >> 18) & 0x3FFCu) : ((v >> 2) & 0x3FFCu);
-        const uint32_t la = (c & 1) ? ((v >> 15) & 0x3FFCu) : ((v << 1) & 0x3FFCu);
-        hv[i] = lds_word(kDqOffHi + ha);
-        lv[i] = lds_word(kDqOffLo + la);
+      for (int i = 0; i < RT; ++i) {
+        code_lut_words(word(i, c), c & 1, kDqOffHi, kDqOffLo, hv[i], lv[i]);
         if (HAS2) {
           const uint32_t idx = ((c < 4 ? cw1[i].x : cw1[i].y) >> (8 * (c & 3))) & 0xFFu;
           l1[c & 1][i] = __builtin_bit_cast(half8, lut1[idx]);
@@ -225,87 +207,79 @@ __global__ __launch_bounds__(kWgThreads) void wg_kernel(WgArgs A) {
       }
     };
     // E8P value +-(k + 1/2); the code's +-1/4 shift is added per slice below
-    auto build = [&](int i, int c) -> half8 {
-      return __builtin_bit_cast(half8, make_uint4(lut_pair_lo(hv[i]), lut_pair_hi(hv[i]), lut_pair_lo(lv[i]),
-                                                  lut_pair_hi(lv[i])));
-    };
-    half8 a[2][kWgRowTiles];
+    half8 a[2][RT];
     read_luts(0);
 #pragma unroll
-    for (int i = 0; i < kWgRowTiles; ++i) a[0][i] = build(i, 0);
+    for (int i = 0; i < RT; ++i) a[0][i] = code_operand(hv[i], lv[i]);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      // B fragments of step c + kWgAhead (into the ring slot step c - 1 freed)
-      {
-        const int cn = c + kWgAhead;
-        load_b(cn < 8 ? s : s + 1, cn & 7, bring[cn % kWgRing]);
-      }
+      // B fragments of step c + kAhead (into the ring slot step c - 1 freed)
+      load_b(c + kAhead < 8 ? s : s + 1, (c + kAhead) & 7, bring[(c + kAhead) % kRing]);
       if (c < 7) read_luts(c + 1);
-      const half8(&bf)[kWgColTiles] = bring[c % kWgRing];
+      const half8(&bf)[NB] = bring[c % kRing];
 #pragma unroll
-      for (int i = 0; i < kWgRowTiles; ++i) {
+      for (int i = 0; i < RT; ++i) {
 #pragma unroll
-        for (int t = 0; t < kWgColTiles; ++t)
+        for (int t = 0; t < NB; ++t)
           acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[c & 1][i], bf[t], acc[i][t], 0, 0, 0);
         if (HAS2) {
 #pragma unroll
-          for (int t = 0; t < kWgColTiles; ++t)
+          for (int t = 0; t < NB; ++t)
             acc2[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(l1[c & 1][i], bf[t], acc2[i][t], 0, 0, 0);
         }
-        if (c < 7) a[(c + 1) & 1][i] = build(i, c + 1);
+        if (c < 7) a[(c + 1) & 1][i] = code_operand(hv[i], lv[i]);
       }
     }
     // shifts: +-1 per code (its shift bit) times the group sums / 4 -- one
     // MFMA per tile pair for the slice's 8 steps
 #pragma unroll
-    for (int i = 0; i < kWgRowTiles; ++i) {
+    for (int i = 0; i < RT; ++i) {
       const uint32_t wd[4] = {cw[i].x, cw[i].y, cw[i].z, cw[i].w};
       uint32_t sh[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) sh[k] = 0xBC00BC00u ^ ((wd[k] & 0x10001u) * 0x8000u);
       const half8 so = __builtin_bit_cast(half8, make_uint4(sh[0], sh[1], sh[2], sh[3]));
 #pragma unroll
-      for (int t = 0; t < kWgColTiles; ++t)
+      for (int t = 0; t < NB; ++t)
         acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(so, sgs[t], acc[i][t], 0, 0, 0);
     }
-    }  // wave_on
-    store_codes(p ^ 1, gc);
-    __syncthreads();
   }
 
   // lane (q, r16) holds weight rows 4 q .. 4 q + 3 of tile i for activation
   // row r16 of tile t: four consecutive outputs
 #pragma unroll
-  for (int t = 0; t < kWgColTiles; ++t) {
-    const int b = (kWgWaves * kWgColTiles * ct + w + kWgWaves * t) * 16 + r16;
+  for (int t = 0; t < NB; ++t) {
+    const int b = (NB * (WC * ct + w % WC) + t) * 16 + r16;
     if (b >= A.B) continue;
-    float* yrow = A.y1p + ((size_t)g * A.B + b) * A.m;
+    float* yrow = J.y1p + ((size_t)g * A.B + b) * J.m;
 #pragma unroll
-    for (int i = 0; i < kWgRowTiles; ++i) {
-      const int rb = rt * kWgRowTiles + i;
-      if (rb >= A.RB) continue;
+    for (int i = 0; i < RT; ++i) {
+      const int rb = rb0 + i;
+      if (rb >= J.RB) continue;
       floatx4 v;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = HAS2 ? A.s0 * acc[i][t][j] + A.s1 * acc2[i][t][j] : A.s0 * acc[i][t][j];
+      for (int j = 0; j < 4; ++j) v[j] = HAS2 ? J.s0 * acc[i][t][j] + J.s1 * acc2[i][t][j] : J.s0 * acc[i][t][j];
       *reinterpret_cast<floatx4*>(yrow + rb * 16 + 4 * q) = v;
     }
   }
 }
 
-template <bool HAS2, int CT>
+template <bool HAS2, int NB, int WC>
 int launch_wg(const WgArgs& A, unsigned grid, hipStream_t stream) {
-  static int done = 0;
-  if (!done) {
-    hipFuncAttributes fa{};
-    QS_HIP(hipFuncGetAttributes(&fa, (const void*)wg_kernel<HAS2, CT>));
-    QS_REQUIRE(fa.sharedSizeBytes == 0, "wg_kernel must not use static LDS");
-    done = 1;
-  }
-  hipLaunchKernelGGL((wg_kernel<HAS2, CT>), dim3(grid), dim3(kWgThreads), kWgLds, stream, A);
+  hipLaunchKernelGGL((wg_kernel<HAS2, NB, WC>), dim3(grid), dim3(kWgThreads), kWgLds, stream, A);
   QS_LAUNCHED("wg_kernel");
   return QS_OK;
 }
-
+template <bool HAS2>
+int launch_wg(const WgArgs& A, int cols, unsigned grid, hipStream_t stream) {
+  switch (cols) {
+    case 2: return launch_wg<HAS2, 2, 1>(A, grid, stream);
+    case 3: return launch_wg<HAS2, 3, 1>(A, grid, stream);
+    case 4: return launch_wg<HAS2, 4, 1>(A, grid, stream);
+    case 6: return launch_wg<HAS2, HAS2 ? 6 : 3, HAS2 ? 1 : 2>(A, grid, stream);
+    default: return launch_wg<HAS2, HAS2 ? 8 : 4, HAS2 ? 1 : 2>(A, grid, stream);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Producer / consumer variant for long single-stage batches
@@ -561,89 +535,81 @@ int launch_wp(const WgArgs& A, unsigned grid, hipStream_t stream) {
 
 }  // namespace
 
-int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
-  const int64_t cols = 16 * kWgWaves * wg_ct(B, has2);
-  const int64_t tiles = ((m / 16 + kWgRowTiles - 1) / kWgRowTiles) * ((B + cols - 1) / cols);
+// Work-group tiles of one linear (128 weight rows by the work-group's activation rows).
+static int64_t wide_tiles(int64_t m, int64_t B, bool has2) {
+  const int64_t cols = use_wp(B, has2) ? 256 : 16 * wg_cols(B);
+  return ((m / 16 + kWgRowTiles - 1) / kWgRowTiles) * ((B + cols - 1) / cols);
+}
+static int groups_within(int64_t tiles, int64_t n, int64_t limit) {
   const int64_t S = n / 256;
-  int64_t g = 1;  // as many groups as fit in one round of work-groups
-  while (g < kWideMaxGroups && g < S && tiles * (g + 1) <= ncu) ++g;
+  int64_t g = 1;
+  while (g < kWideMaxGroups && g < S && tiles * (g + 1) <= limit) ++g;
   return (int)g;
+}
+
+int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
+  const int64_t tiles = wide_tiles(m, B, has2);
+  int g = groups_within(tiles, n, ncu);
+  // up to 128 rows a second work-group per CU, while the partial sums stay few
+  if (B <= 16 * kWgMaxCols) {
+    const int g2 = groups_within(tiles, n, 2 * ncu), most = (int)(kWgPartialBytes / (B * m * 4));
+    if (g2 > g && most > g) g = g2 < most ? g2 : most;
+  }
+  return g;
 }
 
 int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu) {
-  if (count < 2 || wg_ct(B, false) != 4) return 0;
-  const int64_t cols = 16 * kWgWaves * 4;
-  const int64_t tiles = ((m / 16 + kWgRowTiles - 1) / kWgRowTiles) * ((B + cols - 1) / cols) * count;
-  if (tiles > ncu) return 0;
-  const int64_t S = n / 256;
-  int64_t g = 1;
-  while (g < kWideMaxGroups && g < S && tiles * (g + 1) <= ncu) ++g;
-  return (int)g;
+  if (count < 2 || !use_wp(B, false)) return 0;
+  const int64_t tiles = wide_tiles(m, B, false) * count;
+  return tiles > ncu ? 0 : groups_within(tiles, n, ncu);
 }
 
 namespace {
-WgArgs wide_args(const WideMfma& G) {
-  const int CT = wg_ct(G.B, G.codes1 != nullptr);
-  WgArgs A{};
-  A.codes0 = static_cast<const uint16_t*>(G.codes0);
-  A.codes1 = static_cast<const uint8_t*>(G.codes1);
-  A.x2f = G.x2f;
-  A.sgf = G.sgf;
-  A.y1p = G.y1p;
-  A.m = (int)G.m;
-  A.B = G.B;
-  A.S = (int)(G.n / 256);
-  A.RB = (int)(G.m / 16);
+int wide_args(const WideMfma* G, int count, WgArgs& A) {
+  const bool has2 = G[0].codes1 != nullptr;
+  const int cols = use_wp(G[0].B, has2) ? 256 : 16 * wg_cols(G[0].B);
+  A.m = (int)G[0].m;
+  A.B = G[0].B;
+  A.S = (int)(G[0].n / 256);
+  A.RB = (int)(G[0].m / 16);
   A.nrt = (A.RB + kWgRowTiles - 1) / kWgRowTiles;
-  A.nct = (G.B + 16 * kWgWaves * CT - 1) / (16 * kWgWaves * CT);
-  A.SGk = G.SGk;
-  A.spg = (A.S + G.SGk - 1) / G.SGk;
-  A.s0 = G.s0;
-  A.s1 = G.s1;
-  A.njobs = 1;
-  A.job[0] = WpJob{A.codes0, A.x2f, A.y1p, A.s0};
-  return A;
-}
-int check_wide(const WideMfma& G) {
-  QS_REQUIRE(G.m % 16 == 0 && G.n % 256 == 0 && G.B >= 1, "wide GEMM: m %% 16, n %% 256");
-  QS_REQUIRE(G.SGk >= 1 && G.SGk <= kWideMaxGroups, "wide GEMM: 1..%d slice groups", kWideMaxGroups);
-  QS_REQUIRE(G.m * G.n / 4 < ((int64_t)1 << 40), "wide GEMM: codes too large");
+  A.nct = (G[0].B + cols - 1) / cols;
+  A.SGk = G[0].SGk;
+  A.spg = (A.S + A.SGk - 1) / A.SGk;
+  A.njobs = count;
+  int64_t tiles = 0;
+  for (int j = 0; j < count; ++j) {
+    const WideMfma& F = G[j];
+    QS_REQUIRE(F.m % 16 == 0 && F.n % 256 == 0 && F.B >= 1, "wide GEMM: m %% 16, n %% 256");
+    QS_REQUIRE(F.SGk >= 1 && F.SGk <= kWideMaxGroups, "wide GEMM: 1..%d slice groups", kWideMaxGroups);
+    QS_REQUIRE(F.m * F.n / 4 < ((int64_t)1 << 40), "wide GEMM: codes too large");
+    QS_REQUIRE(F.n == G[0].n && F.B == A.B && (F.codes1 != nullptr) == has2, "wide GEMM: linears of one operand width");
+    const int RB = (int)(F.m / 16), nrt = (RB + kWgRowTiles - 1) / kWgRowTiles;
+    A.job[j] = WpJob{static_cast<const uint16_t*>(F.codes0), F.x2f, F.y1p, F.s0, static_cast<const uint8_t*>(F.codes1),
+                     F.sgf, F.s1, (int)F.m, RB, nrt, F.SGk, (A.S + F.SGk - 1) / F.SGk, (int)tiles};
+    tiles += (int64_t)nrt * A.nct * F.SGk;
+    QS_REQUIRE(tiles < ((int64_t)1 << 30), "wide GEMM: grid too large");
+  }
+  A.tiles = (int)tiles;
   return QS_OK;
 }
 }  // namespace
 
-int launch_linear_wide_mfma(const WideMfma& G, hipStream_t stream) {
-  int rc = check_wide(G);
+int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream) {
+  QS_REQUIRE(count >= 1 && count <= QS_MAX_GROUP, "wide GEMM: 1..%d linears", QS_MAX_GROUP);
+  WgArgs A{};
+  const int rc = wide_args(G, count, A);
   if (rc) return rc;
-  const bool has2 = G.codes1 != nullptr;
-  const int CT = wg_ct(G.B, has2);
-  const WgArgs A = wide_args(G);
-  const int64_t tiles = (int64_t)A.nrt * A.nct * A.SGk;
-  QS_REQUIRE(tiles < ((int64_t)1 << 30), "wide GEMM: grid too large");
-  const int64_t grid = (tiles + 7) / 8 * 8;  // XCD-contiguous tile order (see wg_kernel)
-  const unsigned g = (unsigned)grid;
-  if (has2) return CT == 1 ? launch_wg<true, 1>(A, g, stream) : launch_wg<true, 2>(A, g, stream);
-  if (CT == 4) return launch_wp(A, g, stream);  // 256 activation rows per work-group, as wp_kernel's
-  return CT == 1 ? launch_wg<false, 1>(A, g, stream)
-                 : CT == 2 ? launch_wg<false, 2>(A, g, stream) : launch_wg<false, 4>(A, g, stream);
+  const unsigned grid = (unsigned)((A.tiles + 7) / 8 * 8);  // XCD-contiguous tile order (see wg_kernel)
+  const bool has2 = G[0].codes1 != nullptr;
+  if (use_wp(A.B, has2)) {
+    for (int j = 1; j < count; ++j)
+      QS_REQUIRE(G[j].m == G[0].m && G[j].SGk == G[0].SGk, "wide GEMM: one shape beyond %d rows", 16 * kWgMaxCols);
+    return launch_wp(A, grid, stream);
+  }
+  return has2 ? launch_wg<true>(A, wg_cols(A.B), grid, stream) : launch_wg<false>(A, wg_cols(A.B), grid, stream);
 }
 
-int launch_linear_wide_group(const WideMfma* G, int count, hipStream_t stream) {
-  QS_REQUIRE(count >= 1 && count <= QS_MAX_GROUP, "wide GEMM group: 1..%d linears", QS_MAX_GROUP);
-  for (int j = 0; j < count; ++j) {
-    const int rc = check_wide(G[j]);
-    if (rc) return rc;
-    QS_REQUIRE(G[j].m == G[0].m && G[j].n == G[0].n && G[j].B == G[0].B && G[j].SGk == G[0].SGk &&
-                   G[j].codes1 == nullptr && wg_ct(G[j].B, false) == 4,
-               "wide GEMM group: one shape, one stage, more than %d rows", 16 * kWgWaves * 2);
-  }
-  WgArgs A = wide_args(G[0]);
-  A.njobs = count;
-  for (int j = 0; j < count; ++j)
-    A.job[j] = WpJob{static_cast<const uint16_t*>(G[j].codes0), G[j].x2f, G[j].y1p, G[j].s0};
-  const int64_t tiles = (int64_t)A.nrt * A.nct * A.SGk * count;
-  QS_REQUIRE(tiles < ((int64_t)1 << 30), "wide GEMM: grid too large");
-  return launch_wp(A, (unsigned)((tiles + 7) / 8 * 8), stream);
-}
+bool wide_shares_launch(int64_t B, bool has2) { return !use_wp(B, has2); }
 
 }  // namespace qs
