@@ -124,13 +124,13 @@ def ptr(t):
 
 
 def stream_of(t):
-    return _vp(torch.cuda.current_stream(t.device).cuda_stream)
+    return _vp(torch._C._cuda_getCurrentRawStream(t.get_device()))  # torch.cuda.current_stream's handle alone
 
 
 def require_gpu(*tensors, what="quipsharp_amd"):
     """Every compute path runs on the GPU; CPU tensors are rejected, not emulated."""
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"{what} runs on the GPU (MI355X / gfx950); got a tensor on {t.device}")
 
 

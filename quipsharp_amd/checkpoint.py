@@ -10,7 +10,6 @@ matvec kernels in the activation dtype (bf16/fp16/fp32) without a dense
 weight.  ``save_quantized_checkpoint`` / ``load_quantized_checkpoint`` read
 and write the reference's format (state dict + manifest).
 """
-import ctypes
 import json
 import warnings
 import weakref
@@ -19,11 +18,13 @@ from pathlib import Path
 import torch
 from torch import nn, Tensor
 
+from . import _lib
 from .codebooks.e8_1bit import E8OneBitCodebook
 from .codebooks.e8p import E8PCodebook
+from .hadamard import kron_factor
 from .incoherence import IncoherenceSigns, KronSigns
 from .quantize import (PackedCodes, QuantizedLayer, RVQCodebookAdapter, _forward_params, decode_matvec,
-                       forward_packed)
+                       forward_packed, pack_signs, sign_bits_ok)
 from .rfft import RFFTPhases
 from .rvq import RVQStage, fit_residual_stage_scale, fit_stage_scale
 
@@ -137,14 +138,15 @@ class QuantizedLinear(nn.Module):
     def packed(self, kinds):
         # the tensor's identity and version too: a buffer replaced by
         # assignment can reuse a freed block's address
-        key = (id(self.codes), self.codes.data_ptr(), self.codes._version, self.codes.device, tuple(kinds))
+        codes = self.codes
+        key = (id(codes), codes.data_ptr(), codes._version, codes.device, tuple(kinds))
         if self._packed is None or self._packed_key != key:
-            if self.codes.is_cuda and torch.cuda.is_current_stream_capturing():
+            if codes.is_cuda and torch.cuda.is_current_stream_capturing():
                 raise RuntimeError(
                     "QuantizedLinear: the first forward after the module is built, moved, cast or loaded packs "
                     "the codes and reads the scale on the host, which HIP graph capture does not allow: run one "
                     "forward outside capture first")
-            self._packed = PackedCodes(self.codes, self.out_features, self.in_features, kinds)
+            self._packed = PackedCodes(codes, self.out_features, self.in_features, kinds)
             self._packed_key = key
             self._scale_f = float(self.scale.item())
         return self._packed
@@ -176,17 +178,17 @@ class QuantizedLinear(nn.Module):
         takes them (quantize.sign_bits_ok; without x: both sizes on the chunk
         scheme), else the fp32 vectors.  Packed once per sign buffer, outside
         graph capture."""
-        from .quantize import sign_bits_ok
-        su, sv = self._fp32("su"), self._fp32("sv")
+        su_t, sv_t = self.su, self.sv
+        su = su_t if su_t.dtype == torch.float32 else self._fp32("su")
+        sv = sv_t if sv_t.dtype == torch.float32 else self._fp32("sv")
         m, n = self.out_features, self.in_features
         ok = sign_bits_ok(x, m, n) if x is not None else all(d % 256 == 0 and d <= 12288 for d in (m, n))
         if not ok:
             return su, sv
-        key = (id(self.su), self.su.data_ptr(), self.su._version, id(self.sv), self.sv.data_ptr(), self.sv._version)
+        key = (id(su_t), su_t.data_ptr(), su_t._version, id(sv_t), sv_t.data_ptr(), sv_t._version)
         if getattr(self, "_bits_key", None) != key:
             if torch.cuda.is_current_stream_capturing():
                 return su, sv
-            from .quantize import pack_signs
             self._bits = (pack_signs(su), pack_signs(sv))
             self._bits_key = key
         return self._bits
@@ -224,23 +226,23 @@ class QuantizedLinear(nn.Module):
                     if lin is not self:
                         lin._sib_out = (ref, x._version, y)
                 return outs[sib.index(self)]
-        return self._forward_one(x)
+        return self._forward_one(x, (packed, s0, s1))
 
-    def _forward_one(self, x: Tensor) -> Tensor:
-        """This linear alone (RHT / Kronecker transforms)."""
+    def _parts(self):
+        """(packed codes, stage scales) of a forward."""
         kinds, s0, s1 = _forward_params(self.codebook, self.num_stages)
-        packed = self.packed(kinds)
-        ws = self._workspace(x, packed)
+        return self.packed(kinds), s0, s1
+
+    def _forward_one(self, x: Tensor, parts=None) -> Tensor:
+        """This linear alone (RHT / Kronecker transforms)."""
+        packed, s0, s1 = parts or self._parts()
         su, sv = self.signs(x)
         return forward_packed(x, packed, su, sv, s0, s1, self._scale_f, bias=self._fp32("bias"),
-                              out_dtype=x.dtype, workspace=ws)
+                              out_dtype=x.dtype, workspace=self._workspace)
 
-    def _workspace(self, x, packed):
-        from . import _lib
-        rows = x.numel() // x.shape[-1] if x.dim() else 1
-        need = _lib.lib().qs_linear_workspace_bytes(self.out_features, self.in_features, max(rows, 1), packed.layout)
-        if self._ws is None or self._ws.numel() < need or self._ws.device != x.device:
-            self._ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)
+    def _workspace(self, need: int, device) -> Tensor:
+        if self._ws is None or self._ws.numel() < need or self._ws.device != device:
+            self._ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=device)
         return self._ws
 
 
@@ -248,22 +250,28 @@ def groupable(x: Tensor, linears) -> bool:
     """True when the library's grouped forward covers these linears for x (rht
     / krht transforms, n a multiple of 256 with n / p >= 256, tiled code
     layout, the same number of stages)."""
-    from . import _lib
-    from .hadamard import kron_factor
+    return _group_parts(x, linears) is not None
+
+
+def _group_parts(x: Tensor, linears):
+    """The linears' packed codes and stage scales for a grouped forward of x, or
+    None where groupable() is false."""
     n = x.shape[-1] if x.dim() else 0
     rows = x.numel() // n if n else 0
     fn = kron_factor(n) if n else None
     if not (1 <= len(linears) <= _lib.QS_MAX_GROUP and rows >= 1 and n % 256 == 0
             and fn is not None and n // fn[0] >= 256):
-        return False
+        return None
     if not all(isinstance(l, QuantizedLinear) and l.transform_kind in ("rht", "krht") and l.in_features == n
                and l.num_stages == linears[0].num_stages for l in linears):
-        return False
+        return None
+    parts = []
     for l in linears:
-        kinds, _, _ = _forward_params(l.codebook, l.num_stages)
-        if l.packed(kinds).layout != _lib.QS_LAYOUT_TILED:
-            return False
-    return True
+        part = l._parts()
+        if part[0].layout != _lib.QS_LAYOUT_TILED:
+            return None
+        parts.append(part)
+    return parts
 
 
 def link_sibling_linears(model: nn.Module) -> int:
@@ -296,10 +304,11 @@ def grouped_forward(x: Tensor, linears):
     forward per linear above) and one call each otherwise.  Each output equals ``lin(x)``.  No counterpart in the
     reference, which calls the linears one by one; meant for callers that own
     several linears of one input (q/k/v, gate/up)."""
-    if not groupable(x, linears):
+    parts = _group_parts(x, linears)
+    if parts is None:
         return [l._forward_one(x) if isinstance(l, QuantizedLinear) and l.transform_kind != "rfft" else l(x)
                 for l in linears]
-    return _grouped(x, linears)
+    return _grouped(x, linears, parts=parts)
 
 
 def run_preop(x: Tensor, pre: dict) -> Tensor:
@@ -347,12 +356,10 @@ def grouped_forward_pre(x: Tensor, linears, pre: dict):
     return grouped_forward(run_preop(x, pre), linears)
 
 
-def _grouped(x: Tensor, linears, pre: dict = None):
-    """The grouped forward proper, for linears that groupable() accepts."""
-    from . import _lib
+def _grouped(x: Tensor, linears, pre: dict = None, parts=None):
+    """The grouped forward proper, for linears that groupable() accepts
+    (``parts``: what _group_parts returned for them)."""
     from .quantize import forward_packed_group
-    n = x.shape[-1]
-    rows = x.numel() // n
     jobs = []
     signs = [l.signs(x) for l in linears]
     if not all(su.dtype == torch.int32 for su, _ in signs):
@@ -360,17 +367,18 @@ def _grouped(x: Tensor, linears, pre: dict = None):
         # (a member whose out_features is off the chunk scheme, or whose bits are
         # stale under capture, has fp32 signs)
         signs = [(l._fp32("su"), l._fp32("sv")) for l in linears]
-    for l, (su, sv) in zip(linears, signs):
-        kinds, s0, s1 = _forward_params(l.codebook, l.num_stages)
-        jobs.append((l.packed(kinds), su, sv, s0, s1, l._scale_f, l._fp32("bias")))
+    for l, (su, sv), (packed, s0, s1) in zip(linears, signs, parts or [l._parts() for l in linears]):
+        jobs.append((packed, su, sv, s0, s1, l._scale_f, l._fp32("bias")))
     lead = linears[0]
-    ms = (ctypes.c_int64 * len(linears))(*[l.out_features for l in linears])
-    need = _lib.lib().qs_linear_group_workspace_bytes(n, rows, len(linears), ms)
-    ws = getattr(lead, "_group_ws", None)
-    if ws is None or ws.numel() < need or ws.device != x.device:
-        ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)  # zeroed once, reused
-        lead._group_ws = ws
-    return forward_packed_group(x, jobs, out_dtype=x.dtype, workspace=ws, pre=pre)
+
+    def workspace(need, device):
+        ws = getattr(lead, "_group_ws", None)
+        if ws is None or ws.numel() < need or ws.device != device:
+            ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=device)  # zeroed once, reused
+            lead._group_ws = ws
+        return ws
+
+    return forward_packed_group(x, jobs, out_dtype=x.dtype, workspace=workspace, pre=pre)
 
 
 def replace_with_quantized_linear_(parent: nn.Module, attr: str, layer: QuantizedLayer, codebook,

@@ -42,7 +42,7 @@ _KRON_CACHE = {}
 def hartley_matrix(p: int, device=None) -> Tensor:
     """Normalized discrete Hartley matrix cas(2 pi a b / p) / sqrt(p), fp32.
     Symmetric and orthogonal, hence an involution."""
-    key = (p, str(device))
+    key = (p, device if isinstance(device, torch.device) else str(device))
     K = _KRON_CACHE.get(key)
     if K is None:
         a = torch.arange(p, dtype=torch.int64)

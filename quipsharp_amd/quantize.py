@@ -254,11 +254,13 @@ def forward_packed(x: Tensor, packed: PackedCodes, su: Tensor, sv: Tensor, s0: f
                    out: Tensor = None, mv_events=None) -> Tensor:
     """y = su (.) T_m(layer_scale * W_hat @ T_n(sv (.) x)) + bias for x (..., n),
     computed in the library (fp32 accumulation; output in ``out_dtype``,
-    default x.dtype)."""
+    default x.dtype).  ``workspace``: a tensor, or a function (bytes, device) that
+    returns one of at least that size, called once."""
     _lib.require_gpu(x, su, sv, bias, what="linear forward")
     m, n = packed.m, packed.n
     if x.shape[-1] != n:
         raise ValueError(f"expected last dim {n}, got {x.shape[-1]}")
+    grow, workspace = (workspace, None) if callable(workspace) else (None, workspace)
     bits = check_linear_args(x, m, n, su, sv, bias, out, workspace)
     if packed.codes0.device != x.device:
         raise ValueError(f"codes are on {packed.codes0.device}, x on {x.device}")
@@ -280,7 +282,7 @@ def forward_packed(x: Tensor, packed: PackedCodes, su: Tensor, sv: Tensor, s0: f
     need = lib.qs_linear_workspace_bytes(m, n, B, packed.layout)
     if workspace is None or workspace.numel() < need:
         # zero-initialised: the first 256 bytes are the fused kernel's counter
-        workspace = torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)
+        workspace = grow(need, x.device) if grow else torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)
     _lib.check(lib.qs_linear_forward(
         _lib.ptr(x2), _lib.dtype_code(x2.dtype), x2.stride(0), B, n, m, _lib.ptr(packed.codes0),
         _lib.ptr(packed.codes1), packed.kind1, packed.layout | (_lib.QS_SIGNS_BITS if bits else 0),
@@ -338,6 +340,7 @@ def forward_packed_group(x: Tensor, linears, out_dtype=None, workspace: Tensor =
     Tensor or None, "eps": float}`` (input = RMSNorm(x + delta), x + delta
     written to h_out); 1-2 rows, or 3-16 on the chunk scheme (``pre_ok``),
     bit-identical to ``qs_dec_rmsnorm`` followed by the grouped forward."""
+    grow, workspace = (workspace, None) if callable(workspace) else (None, workspace)
     count = len(linears)
     if not 1 <= count <= _lib.QS_MAX_GROUP:
         raise ValueError(f"1..{_lib.QS_MAX_GROUP} linears per group, got {count}")
@@ -386,7 +389,7 @@ def forward_packed_group(x: Tensor, linears, out_dtype=None, workspace: Tensor =
     ms = (ctypes.c_int64 * count)(*[lin[0].m for lin in linears])
     need = lib.qs_linear_group_workspace_bytes(n, B, count, ms)
     if workspace is None or workspace.numel() < need:
-        workspace = torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)
+        workspace = grow(need, x.device) if grow else torch.zeros(max(need, 256), dtype=torch.uint8, device=x.device)
     if pre is not None:
         op = _pre_struct(x2, pre, n)
         _lib.check(lib.qs_linear_forward_group_pre(
