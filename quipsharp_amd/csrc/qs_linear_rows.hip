@@ -22,8 +22,10 @@
 // the short batches (qs_linear_batched.hip, qs_linear_big.hip) spread one row
 // over 16 waves with three barriers, which is the shorter chain for a few rows
 // but leaves a CU waiting when there are many.
-// Rows longer than 16 chunks are read once per group of 16 slices; the work-
-// groups of a row tile run on one XCD, whose L2 serves the repeats.
+// Rows longer than 16 chunks are read once per group of 16 slices.  On the input
+// side the work-groups of a row tile run on one XCD, whose L2 serves the repeats;
+// on the output side, with four bytes an element, one work-group takes all the
+// groups of a row.
 //
 // Measured (bf16, sum over a layer's launches, per-row kernels -> this):
 //   input, Llama-2-7B   130 rows 35 -> 37 us, 200 39 -> 37, 512 66 -> 45, 2000 212 -> 116
@@ -31,10 +33,11 @@
 //   output beyond 12288 (Llama-3-8B gate + up) 130 rows 29 -> ~46 us, 320 57 -> ~42, 2000 360 -> ~150
 //   output up to 12288 (Llama-2-7B) 512 rows 62 -> 86 us, 2000 201 -> 231: not taken
 // so the input runs here from kRowsInMin rows, the output from kRowsOutMin rows
-// beyond 12288.  The output kernel is bound by its reads of fp32 partial sums,
-// once per group of 16 slices through the L1's 64 bytes a clock, and by
-// splitting them each time; up to 12288 qs_linear_batched.hip's by_kernel reads
-// them once.
+// beyond 12288.  The output kernel reads the fp32 partial sums once per group
+// of 16 slices and splits them each time; up to 12288 qs_linear_batched.hip's
+// by_kernel reads them once.  Groups of a row in one work-group instead of one
+// each (the layer's calls, 2 bits): Qwen2.5-7B 2000 rows 1382 -> 1333 us, 4000
+// 2585 -> 2454, Qwen3-32B 2000 2618 -> 2573, Llama-3-8B 4000 2097 -> 2078.
 #include "qs_forward_dev.h"
 #include "qs_linear_dev.h"
 
@@ -57,10 +60,10 @@ __device__ __forceinline__ uint32_t perm_hi(uint32_t hi, uint32_t lo) {
 
 // Rows 16 k .. 16 k + 15 of M (zero past S) as two 16-bit planes whose sum is
 // the entry to 16 bits or more: truncated bf16, or fp16 for F16.
-template <bool F16>
+template <bool F16, int NT = kRowsThreads>
 __device__ __forceinline__ void build_m16(uint16_t* Mh, uint16_t* Ml, int k, int S, int Spad, int lsh, int p,
                                           const float* K, int tid) {
-  for (int e = tid; e < 16 * Spad; e += kRowsThreads) {
+  for (int e = tid; e < 16 * Spad; e += NT) {
     const int rr = e / Spad, c = e - rr * Spad;
     const int r = 16 * k + rr;
     const float v = r < S && c < S ? mmat(r, c, lsh, p, K) : 0.0f;
@@ -420,10 +423,19 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
 // ---------------------------------------------------------------------------
 // output transform
 // ---------------------------------------------------------------------------
+// A work-group's 8 waves take turns at the pairs of its rows and groups of 16
+// slices, so that the groups of one row are in work at one time and its partial
+// sums, which every group needs whole, come from memory once and then from the
+// L1 and L2.  (Work-groups with one group each drifted apart: five groups of a
+// 18944 wide row fetched 3 GB instead of 0.6.)  M of all the groups is in LDS,
+// and the signs as bits; signs that are not +-1 and the bias are read as needed.
+constexpr int kWyThreads = 512;
+constexpr int kWyWaves = kWyThreads / 64;
+constexpr int kMaxGroups16 = kRowsMaxS / 16;
 struct WyJob {
-  RowsSlot at;
+  int wg0, per;      // first work-group, work-groups
   const float* y1p;  // [SG][B][m]
-  int SG, m, S, lsh, pm;
+  int SG, m, S, lsh, pm, ngrp;
   const float* Km;
   float scale;       // of the transform, times the layer's
   const float* xmul;
@@ -432,41 +444,58 @@ struct WyJob {
   void* y;
   int64_t ldy;
   int wide;          // y rows start on 16 bytes
+  int bias_wide;     // the bias starts on 16 bytes
 };
 struct WyArgs {
   int B, y_dtype, njobs;
   WyJob job[QS_MAX_GROUP];
 };
-constexpr int kSuStr = 256 + 4;  // signs and bias per slice
 constexpr int kYStr = 256 + 8;  // outputs per slice of a row (16-byte words of two rows in distinct banks)
 struct WyLds {
-  uint16_t Mh[16 * kRowsMStr], Ml[16 * kRowsMStr];
-  float su[16 * kSuStr], bias[16 * kSuStr];  // of this work-group's slices
-  uint16_t out[kRowsWaves][16 * kYStr];
+  uint32_t sign[kRowsMaxS * 8];  // bit t % 32 of word t / 32: column t is negative
+  uint16_t out[kWyWaves][16 * kYStr];
+  uint16_t M[kMaxGroups16][2][16 * kRowsMStr];  // as many groups as the launch has
 };
+constexpr size_t wy_lds(int groups) {
+  return sizeof(WyLds) - (size_t)(kMaxGroups16 - groups) * 2 * 16 * kRowsMStr * sizeof(uint16_t);
+}
+static_assert(wy_lds(kMaxGroups16) <= 160 * 1024, "LDS budget");
 
 // LO: a job's M has a second plane.
 template <bool SB, bool LO>
-__global__ __launch_bounds__(kRowsThreads, 2) void wy_kernel(WyArgs A) {
-  __shared__ WyLds D;
+__global__ __launch_bounds__(kWyThreads) void wy_kernel(WyArgs A) {
+  extern __shared__ __attribute__((aligned(16))) char wy_sm[];
+  WyLds& D = *reinterpret_cast<WyLds*>(wy_sm);
+  __shared__ int odd_sign;
   const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
   int g = 0;
 #pragma unroll
   for (int j = 1; j < QS_MAX_GROUP; ++j)
-    if (j < A.njobs && (int)blockIdx.x >= A.job[j].at.wg0) g = j;
+    if (j < A.njobs && (int)blockIdx.x >= A.job[j].wg0) g = j;
   const WyJob J = A.job[g];
   const int S = J.S, nkb = (S + 31) >> 5;
-  int k, turn;
-  rows_place((int)blockIdx.x - J.at.wg0, J.at, k, turn);
-  build_m16<false>(D.Mh, D.Ml, k, S, 32 * nkb, J.lsh, J.pm, J.Km, tid);
-  for (int i = tid; i < 16 * 256; i += kRowsThreads) {
-    const int o = 4096 * k + i, at = o < J.m ? o : J.m - 1;
-    const int to = (i >> 8) * kSuStr + (i & 255);
-    if constexpr (SB) D.su[to] = (reinterpret_cast<const uint32_t*>(J.su)[at >> 5] >> (at & 31)) & 1 ? -1.0f : 1.0f;
-    else D.su[to] = J.su[at];
-    D.bias[to] = J.bias ? J.bias[at] : 0.0f;
-  }
+  const int wg = (int)blockIdx.x - J.wg0;
+  for (int k = 0; k < J.ngrp; ++k)
+    build_m16<false, kWyThreads>(D.M[k][0], D.M[k][1], k, S, 32 * nkb, J.lsh, J.pm, J.Km, tid);
+  if (tid == 0) odd_sign = 0;
   __syncthreads();
+  bool odd = false;
+  for (int i = tid; i < 8 * S; i += kWyThreads) {
+    uint32_t w = 0;
+    if constexpr (SB) {
+      w = reinterpret_cast<const uint32_t*>(J.su)[i];
+    } else {
+      for (int t = 0; t < 32; ++t) {
+        const float f = J.su[32 * i + t];
+        odd = odd || fabsf(f) != 1.0f;
+        w |= (f < 0.0f ? 1u : 0u) << t;
+      }
+    }
+    D.sign[i] = w;
+  }
+  if (odd) odd_sign = 1;
+  __syncthreads();
+  const bool plain = SB || odd_sign == 0;
   // columns 64 x + 4 r16 .. + 3 of the eight chunks of k-step kb (256 consecutive
   // bytes per 16 lanes), requested one block ahead
   float4 nx[8];
@@ -478,15 +507,13 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wy_kernel(WyArgs A) {
       nx[i] = *reinterpret_cast<const float4*>(src + 256 * (c < S ? c : S - 1));
     }
   };
-  const int row = tid >> 6;
-  const int turns = (A.B + 32 * kRowsWaves - 1) / (32 * kRowsWaves) * 32;
-  auto row_of = [&](int t) { return rows_first(t) + row < A.B ? rows_first(t) + row : A.B - 1; };
-  if (turn < turns) request(row_of(turn), 0, 0, 0);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int turns = (A.B - wg + J.per - 1) / J.per * J.ngrp;
+  if (wave < turns) request(wg + wave / J.ngrp * J.per, 0, 0, 0);
 
-  for (; turn < turns; turn += J.at.per) {  // no barrier follows
-    const int b = rows_first(turn) + row;
-    if (b >= A.B) continue;
-    const int next = turn + J.at.per < turns ? row_of(turn + J.at.per) : b;
+  for (int turn = wave; turn < turns; turn += kWyWaves) {  // no barrier follows
+    const int i0 = turn / J.ngrp, k = turn - i0 * J.ngrp, b = wg + i0 * J.per;
+    const int next = turn + kWyWaves < turns ? wg + (turn + kWyWaves) / J.ngrp * J.per : b;
     floatx4 acc[4][4];
 #pragma unroll
     for (int x = 0; x < 4; ++x)
@@ -494,8 +521,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wy_kernel(WyArgs A) {
       for (int u = 0; u < 4; ++u) acc[x][u] = (floatx4){0.f, 0.f, 0.f, 0.f};
     for (int kb = 0; kb < nkb; ++kb) {
       const int c0 = 32 * kb + 8 * q;
-      const bf16x8 ah = *reinterpret_cast<const bf16x8*>(D.Mh + r16 * kRowsMStr + c0);
-      const bf16x8 al = *reinterpret_cast<const bf16x8*>(D.Ml + r16 * kRowsMStr + c0);
+      const bf16x8 ah = *reinterpret_cast<const bf16x8*>(D.M[k][0] + r16 * kRowsMStr + c0);
+      const bf16x8 al = *reinterpret_cast<const bf16x8*>(D.M[k][1] + r16 * kRowsMStr + c0);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         float4 z[8];
@@ -538,14 +565,22 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wy_kernel(WyArgs A) {
     h256_rows<4>(acc);
     const float mul = J.scale * J.xmul[b];
     const int s = 16 * k + r16;
-    uint16_t* stage = D.out[row];
+    uint16_t* stage = D.out[wave];
+    const int col = 256 * (s < S ? s : S - 1);  // slices past S: computed, never stored
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int t0 = 64 * x + 16 * j + 4 * q;
-        const float4 su = *reinterpret_cast<const float4*>(D.su + kSuStr * r16 + t0);
-        const float4 bi = *reinterpret_cast<const float4*>(D.bias + kSuStr * r16 + t0);
+        const uint32_t neg = D.sign[(col + t0) >> 5] >> (t0 & 31);
+        float4 su = make_float4(neg & 1 ? -1.0f : 1.0f, neg & 2 ? -1.0f : 1.0f, neg & 4 ? -1.0f : 1.0f,
+                                neg & 8 ? -1.0f : 1.0f);
+        if (!plain) su = *reinterpret_cast<const float4*>(J.su + col + t0);
+        float4 bi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (J.bias) {
+          const float* p = J.bias + col + t0;
+          bi = J.bias_wide ? *reinterpret_cast<const float4*>(p) : make_float4(p[0], p[1], p[2], p[3]);
+        }
         const float o[4] = {acc[x][0][j] * mul * su.x + bi.x, acc[x][1][j] * mul * su.y + bi.y,
                             acc[x][2][j] * mul * su.z + bi.z, acc[x][3][j] * mul * su.w + bi.w};
         if (A.y_dtype == QS_DTYPE_F32) {
@@ -666,21 +701,25 @@ int launch_wy(const BatchedPass* P, int count, hipStream_t stream) {
   int groups = 0;
   bool odd = false;  // a job without an odd factor has a zero second plane
   for (int g = 0; g < count; ++g) groups += (int)((P[g].m / 256 + 15) / 16), odd = odd || P[g].pm > 1;
-  const int per = rows_per_group(A.B, groups, P[0].ncu);
-  int wg = 0;
+  int wg = 0, most = 1;
   for (int g = 0; g < count; ++g) {
     const BatchedPass& Q = P[g];
     QS_REQUIRE(rows_output_fits(Q) && Q.B == A.B && Q.y_dtype == A.y_dtype && Q.sbits == P[0].sbits,
                "output transform: m %lld (p %d) or mixed rows / dtype / sign format", (long long)Q.m, Q.pm);
     const size_t es = Q.y_dtype == QS_DTYPE_F32 ? 4 : 2;
     const int S = (int)(Q.m / 256), ngrp = (S + 15) / 16;
-    A.job[g] = WyJob{{wg, ngrp, per},
+    // one work-group per CU (by its LDS), dealt by the linears' sizes
+    int per = P[0].ncu * ngrp / groups;
+    per = per < 1 ? 1 : per > A.B ? A.B : per;
+    A.job[g] = WyJob{wg,
+                     per,
                      Q.y1p,
                      Q.SG,
                      (int)Q.m,
                      S,
                      log2_exact(Q.m / Q.pm / 256),
                      Q.pm,
+                     ngrp,
                      Q.Km,
                      inv_sqrt_len(Q.m / Q.pm) * Q.layer_scale,
                      Q.xmul,
@@ -688,17 +727,20 @@ int launch_wy(const BatchedPass* P, int count, hipStream_t stream) {
                      Q.bias,
                      Q.y,
                      Q.ldy,
-                     (reinterpret_cast<uintptr_t>(Q.y) & 15) == 0 && Q.ldy * es % 16 == 0};
-    wg += ngrp * per;
+                     (reinterpret_cast<uintptr_t>(Q.y) & 15) == 0 && Q.ldy * es % 16 == 0,
+                     (reinterpret_cast<uintptr_t>(Q.bias) & 15) == 0};
+    wg += per;
+    most = ngrp > most ? ngrp : most;
   }
-  const dim3 grid((unsigned)wg), block(kRowsThreads);
-  if (P[0].sbits) {
-    if (odd) hipLaunchKernelGGL((wy_kernel<true, true>), grid, block, 0, stream, A);
-    else hipLaunchKernelGGL((wy_kernel<true, false>), grid, block, 0, stream, A);
-  } else {
-    if (odd) hipLaunchKernelGGL((wy_kernel<false, true>), grid, block, 0, stream, A);
-    else hipLaunchKernelGGL((wy_kernel<false, false>), grid, block, 0, stream, A);
-  }
+  const size_t lds = wy_lds(most);
+  auto launch = [&](auto kernel) {
+    QS_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(kWyThreads), lds, stream, A);
+    return (int)QS_OK;
+  };
+  const int rc = P[0].sbits ? (odd ? launch(wy_kernel<true, true>) : launch(wy_kernel<true, false>))
+                            : (odd ? launch(wy_kernel<false, true>) : launch(wy_kernel<false, false>));
+  if (rc) return rc;
   QS_LAUNCHED("wy_kernel");
   return QS_OK;
 }

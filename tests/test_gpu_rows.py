@@ -85,3 +85,35 @@ def test_strides_dtypes_and_row_isolation(dev, m, n):
     assert torch.equal(a, b)
     zero = forward_packed(x, packed, su * 0, sv * 0, 1.0, 0.0, 0.0135, bias)  # signs of a layer not loaded yet
     assert torch.equal(zero, bias.bfloat16().expand(B, m))
+
+
+@pytest.mark.parametrize("m,B,has_bias", [(16384, 320, True), (32768, 323, False), (18944, 600, False)])
+def test_output_factors_that_are_not_signs(dev, m, B, has_bias):
+    """su of other values than +-1 (powers of two: the product is exact), read
+    as they are instead of as bits."""
+    from quipsharp_amd.quantize import forward_packed
+    packed, su, sv, bias, _ = layer(dev, m, 256, m, has_bias)
+    su, sv = su.to(dev), sv.to(dev)
+    x = torch.randn(B, 256, generator=torch.Generator().manual_seed(B)).to(dev)
+    factor = torch.ones(m, device=dev)
+    factor[5::97] = 4.0
+    args = (1.0, 0.0, 0.0135)
+    plain = forward_packed(x, packed, su, sv, *args)
+    assert torch.equal(forward_packed(x, packed, su * factor, sv, *args), plain * factor)
+    if has_bias:
+        b = bias.to(dev).float()
+        odd = torch.empty(m + 1, device=dev)[1:].copy_(b)  # off 16 bytes
+        want = forward_packed(x, packed, su, sv, *args, bias=b)
+        assert torch.equal(forward_packed(x, packed, su, sv, *args, bias=odd), want)
+        assert (want - (plain + b)).abs().max() <= 1e-5 * want.abs().max()
+
+
+def test_group_of_different_long_outputs_equals_single_calls(dev):
+    from quipsharp_amd.quantize import forward_packed, forward_packed_group
+    lins = []
+    for m in (13312, 32768, 14336):
+        packed, su, sv, _, _ = layer(dev, m, 256, m, False)
+        lins.append((packed, su.to(dev), sv.to(dev), 1.0, 0.0, 0.0135, None))
+    x = torch.randn(331, 256, generator=torch.Generator().manual_seed(1)).to(dev)
+    for lin, y in zip(lins, forward_packed_group(x, lins)):
+        assert torch.equal(y, forward_packed(x, *lin))
