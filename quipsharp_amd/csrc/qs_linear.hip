@@ -116,9 +116,8 @@ WsLayout ws_layout(int64_t m, int64_t n, int64_t batch, int layout) {
   if (L.wide) {
     // partial groups of the wide GEMM, or the 16-row passes of the
     // decode-matvec (which also takes this layout)
-    const int g0 = wide_splits(m, n, B, cu_count(), false), g1 = wide_splits(m, n, B, cu_count(), true);
-    const size_t a = (size_t)(g0 > g1 ? g0 : g1) * B, b = (size_t)L.SG * kMaxTileBatch;
-    L.y1p = off; off = align256(off + (a > b ? a : b) * m * 4);
+    const size_t a = wide_partial_bytes(m, n, B, cu_count()), b = (size_t)L.SG * kMaxTileBatch * m * 4;
+    L.y1p = off; off = align256(off + (a > b ? a : b));
   } else {
     const int sgp = L.SG > L.fused.SG ? L.SG : L.fused.SG;
     L.y1p = off; off = align256(off + (size_t)sgp * B * m * 4);

@@ -558,6 +558,19 @@ int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
   return g;
 }
 
+size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu) {
+  size_t most = 0;
+  for (int has2 = 0; has2 < 2; ++has2) {
+    size_t b = (size_t)wide_splits(m, n, B, ncu, has2) * B * m * 4;
+    most = b > most ? b : most;
+    if (B > 16 * kWgMaxCols) continue;
+    b = (size_t)groups_within(wide_tiles(m, B, has2), n, 2 * ncu) * B * m * 4;
+    b = b < (size_t)kWgPartialBytes ? b : (size_t)kWgPartialBytes;
+    most = b > most ? b : most;
+  }
+  return most;
+}
+
 int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu) {
   if (count < 2 || !use_wp(B, false)) return 0;
   const int64_t tiles = wide_tiles(m, B, false) * count;
