@@ -177,52 +177,42 @@ struct WxLds {
   uint4 out[16 * kOutStr];         // a tile's operand words: [slice][word of the slice][row]
 };
 
-// XT: 0 bf16, 1 fp16, 2 fp32 activations; SB: sv is packed sign bits; LO: M
-// has a second plane (an odd factor).
-template <int XT, bool SB, bool LO>
-__global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
-  __shared__ WxLds D;
+// Four consecutive activations (8 or 16 bytes, aligned), exact in fp32.
+template <int XT>
+__device__ __forceinline__ float4 load_x4(const void* x, int64_t at) {
+  if constexpr (XT == 2) return *reinterpret_cast<const float4*>(static_cast<const float*>(x) + at);
+  const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(x) + at);
+  if constexpr (XT == 0)
+    return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xFFFF0000u), __uint_as_float(w.y << 16),
+                       __uint_as_float(w.y & 0xFFFF0000u));
+  const half2v a = __builtin_bit_cast(half2v, w.x), b = __builtin_bit_cast(half2v, w.y);
+  return make_float4((float)a[0], (float)a[1], (float)b[0], (float)b[1]);
+}
+
+// How sv meets the activations: 16-bit ones times +-1 are MFMA operands as they
+// are; fp32 ones, and the products with other multipliers, enter as two bf16
+// planes (truncated, and the remainder rounded), 16 bits or more as in the
+// per-row kernels.  Error against 64 bits, bf16 rows of 3584 with multipliers of
+// 1.03 .. 2.33: 3.3e-3 as one bf16 plane, 2.1e-4 (the fp16 operand's) as two.
+enum class Mul { kExact, kSign, kFactor };
+
+// The rows of a work-group.  A function for each kind of multiplier, so that
+// none takes the others' registers (in one loop the 16-bit rows spilled 50).
+// XT: 0 bf16, 1 fp16, 2 fp32 activations; LO: M has a second plane (an odd factor).
+template <int XT, Mul MUL, bool LO>
+__device__ __forceinline__ void wx_rows(const WxArgs& A, const WxJob& J, WxLds& D, int k, int turn) {
+  constexpr bool kExact = MUL == Mul::kExact;
   const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
   const LaneX lx = lane_x_init();
-  int g = 0;
-#pragma unroll
-  for (int j = 1; j < QS_MAX_GROUP; ++j)
-    if (j < A.njobs && (int)blockIdx.x >= A.job[j].at.wg0) g = j;
-  const WxJob J = A.job[g];
   const int S = A.S, nkb = (S + 31) >> 5;
-  int k, turn;
-  rows_place((int)blockIdx.x - J.at.wg0, J.at, k, turn);
-
-  build_m16<XT == 1>(D.Mh, D.Ml, k, S, 32 * nkb, A.lsh, A.pn, A.Kn, tid);
-  if (tid == 0) D.plain = 1;
+  build_m16<kExact && XT == 1>(D.Mh, D.Ml, k, S, 32 * nkb, A.lsh, A.pn, A.Kn, tid);
   __syncthreads();
-  for (int i = tid; i < 32 * S; i += kRowsThreads) {
-    uint32_t w = 0;
-    if constexpr (SB) {
-      const uint32_t b = reinterpret_cast<const uint8_t*>(J.sv)[i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w |= ((b >> (2 * j)) & 1u) << (15 - j) | ((b >> (2 * j + 1)) & 1u) << (31 - j);
-    } else {
-      const float4 lo = reinterpret_cast<const float4*>(J.sv)[2 * i], hi = reinterpret_cast<const float4*>(J.sv)[2 * i + 1];
-      const float s[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      bool one = true;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        one = one && fabsf(s[e]) == 1.0f;
-        w |= (__float_as_uint(s[e]) >> 31) << ((e & 1 ? 31 : 15) - (e >> 1));
-      }
-      if (!one) D.plain = 0;
-    }
-    D.sign[i] = w;
-  }
-  __syncthreads();
-  const bool plain = SB || D.plain;
   // the operand block of (row b, k-step kb, half th), requested one block ahead
   // (the next row's first one during the last block of a row): with two waves
   // per SIMD nothing else covers the loads
   uint4 nx[8];
   auto request = [&](int b, int kb, int th) __attribute__((always_inline)) {
-    if constexpr (XT != 2) {
+    if constexpr (kExact) {
       const uint16_t* src = static_cast<const uint16_t*>(A.x) + (int64_t)b * A.ldx + 128 * th + 8 * r16;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -253,7 +243,7 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
       const uint4 al = *reinterpret_cast<const uint4*>(D.Ml + r16 * kRowsMStr + c0);
 #pragma unroll
       for (int th = 0; th < 2; ++th) {
-        if constexpr (XT != 2) {
+        if constexpr (kExact) {
           uint32_t d[8][4];
 #pragma unroll
           for (int i = 0; i < 8; ++i) d[i][0] = nx[i].x, d[i][1] = nx[i].y, d[i][2] = nx[i].z, d[i][3] = nx[i].w;
@@ -265,24 +255,9 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
           for (int i = 0; i < 8; ++i) {
             const int c = c0 + i;
             const int at = 32 * (c < S ? c : S - 1) + 16 * th + r16;
-            if (plain) {
-              const uint32_t w = D.sign[at];
+            const uint32_t w = D.sign[at];
 #pragma unroll
-              for (int j = 0; j < 4; ++j) d[i][j] ^= (w << j) & 0x80008000u;
-            } else {  // other multipliers: as the products truncated to 16 bits (bf16) or rounded (fp16)
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const float s0 = J.sv[8 * at + 2 * j], s1 = J.sv[8 * at + 2 * j + 1];
-                if constexpr (XT == 0) {
-                  d[i][j] = perm_hi(__float_as_uint(__uint_as_float(d[i][j] & 0xFFFF0000u) * s1),
-                                    __float_as_uint(__uint_as_float(d[i][j] << 16) * s0));
-                } else {
-                  const half2v h = __builtin_bit_cast(half2v, d[i][j]);
-                  const half2v o = {(_Float16)((float)h[0] * s0), (_Float16)((float)h[1] * s1)};
-                  d[i][j] = __builtin_bit_cast(uint32_t, o);
-                }
-              }
-            }
+            for (int j = 0; j < 4; ++j) d[i][j] ^= (w << j) & 0x80008000u;
             if (32 * kb + 32 > S && c >= S) d[i][0] = d[i][1] = d[i][2] = d[i][3] = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -316,8 +291,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
                 acc[th][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf, __builtin_bit_cast(half8, al), acc[th][u], 0, 0, 0);
             }
           }
-        } else {  // fp32: truncated bf16 and the remainder, four columns at a time
-          const float* src = static_cast<const float*>(A.x) + (int64_t)b * A.ldx + 128 * th + 8 * r16;
+        } else {  // four columns at a time
+          const int64_t src = (int64_t)b * A.ldx + 128 * th + 8 * r16;
 #pragma unroll
           for (int uh = 0; uh < 2; ++uh) {
             uint32_t fh[4][4], fl[4][4];  // [u][pair of chunks]
@@ -327,13 +302,13 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
 #pragma unroll
               for (int i = 0; i < 2; ++i) {
                 const int c = c0 + 2 * i2 + i, cc = c < S ? c : S - 1;
-                const float4 f = *reinterpret_cast<const float4*>(src + 256 * cc + 4 * uh);
+                const float4 f = load_x4<XT>(A.x, src + 256 * cc + 4 * uh);
                 const int at = 32 * cc + 16 * th + r16;
                 v[i][0] = f.x, v[i][1] = f.y, v[i][2] = f.z, v[i][3] = f.w;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                   const int e = 4 * uh + u;
-                  if (plain)
+                  if constexpr (MUL == Mul::kSign)
                     v[i][u] = __uint_as_float(__float_as_uint(v[i][u]) ^
                                               ((D.sign[at] << ((e & 1 ? 0 : 16) + (e >> 1))) & 0x80000000u));
                   else
@@ -346,8 +321,8 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
               for (int u = 0; u < 4; ++u) {
                 const uint32_t a = __float_as_uint(v[0][u]), c = __float_as_uint(v[1][u]);
                 fh[u][i2] = perm_hi(c, a);
-                fl[u][i2] = perm_hi(__float_as_uint(v[1][u] - __uint_as_float(c & 0xFFFF0000u)),
-                                    __float_as_uint(v[0][u] - __uint_as_float(a & 0xFFFF0000u)));
+                fl[u][i2] = f32x2_to_bf16x2(v[0][u] - __uint_as_float(a & 0xFFFF0000u),
+                                            v[1][u] - __uint_as_float(c & 0xFFFF0000u));
               }
             }
 #pragma unroll
@@ -418,6 +393,47 @@ __global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
         *reinterpret_cast<uint4*>(xo + (sl * 512 + (w / kRowsWaves) * 16 + w % kRowsWaves) * 8) = D.out[sl * kOutStr + w];
     }
   }
+}
+
+// SB: sv is packed sign bits.
+template <int XT, bool SB, bool LO>
+__global__ __launch_bounds__(kRowsThreads, 2) void wx_kernel(WxArgs A) {
+  __shared__ WxLds D;
+  const int tid = threadIdx.x;
+  int g = 0;
+#pragma unroll
+  for (int j = 1; j < QS_MAX_GROUP; ++j)
+    if (j < A.njobs && (int)blockIdx.x >= A.job[j].at.wg0) g = j;
+  const WxJob J = A.job[g];
+  const int S = A.S;
+  int k, turn;
+  rows_place((int)blockIdx.x - J.at.wg0, J.at, k, turn);
+
+  if (tid == 0) D.plain = 1;
+  __syncthreads();
+  for (int i = tid; i < 32 * S; i += kRowsThreads) {
+    uint32_t w = 0;
+    if constexpr (SB) {
+      const uint32_t b = reinterpret_cast<const uint8_t*>(J.sv)[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w |= ((b >> (2 * j)) & 1u) << (15 - j) | ((b >> (2 * j + 1)) & 1u) << (31 - j);
+    } else {
+      const float4 lo = reinterpret_cast<const float4*>(J.sv)[2 * i], hi = reinterpret_cast<const float4*>(J.sv)[2 * i + 1];
+      const float s[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      bool one = true;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        one = one && fabsf(s[e]) == 1.0f;
+        w |= (__float_as_uint(s[e]) >> 31) << ((e & 1 ? 31 : 15) - (e >> 1));
+      }
+      if (!one) D.plain = 0;
+    }
+    D.sign[i] = w;
+  }
+  __syncthreads();
+  const bool plain = SB || __builtin_amdgcn_readfirstlane(D.plain) != 0;
+  if (plain) wx_rows<XT, XT == 2 ? Mul::kSign : Mul::kExact, LO>(A, J, D, k, turn);
+  else if constexpr (!SB) wx_rows<XT, Mul::kFactor, LO>(A, J, D, k, turn);
 }
 
 // ---------------------------------------------------------------------------

@@ -117,3 +117,40 @@ def test_group_of_different_long_outputs_equals_single_calls(dev):
     x = torch.randn(331, 256, generator=torch.Generator().manual_seed(1)).to(dev)
     for lin, y in zip(lins, forward_packed_group(x, lins)):
         assert torch.equal(y, forward_packed(x, *lin))
+
+
+def structured_T(v):
+    """T along the last dim of fp64 v (the rows of a dense_T product, for long rows)."""
+    n = v.shape[-1]
+    L = n & -n
+    p = n // L
+    z, h = v.reshape(-1, p, L), 1
+    while h < L:
+        z = z.reshape(-1, p, L // (2 * h), 2, h)
+        z = torch.stack([z[..., 0, :] + z[..., 1, :], z[..., 0, :] - z[..., 1, :]], -2)
+        h *= 2
+    z = z.reshape(-1, p, L) / L ** 0.5
+    i = torch.arange(p, device=v.device, dtype=torch.float64)
+    a = 2 * torch.pi * ((i[:, None] * i) % p) / p
+    return ((a.cos() + a.sin()) / p ** 0.5 @ z).reshape(v.shape)
+
+
+@pytest.mark.parametrize("n", [512, 3584, 11008])
+@pytest.mark.parametrize("B", [159, 160])
+@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1.0), (torch.float16, 1.0), (torch.float16, 3e4),
+                                        (torch.float32, 1.0)])
+def test_input_factors_that_are_not_signs(dev, n, B, dtype, size):
+    """sv of other values than +-1 on both sides of the threshold: the products
+    keep two 16-bit planes, and those beyond fp16's range stay finite."""
+    from quipsharp_amd.codebooks.e8p import _decode
+    from quipsharp_amd.quantize import forward_packed
+    m = 256
+    packed, su, sv, _, codes = layer(dev, m, n, n, False)
+    su, sv = su.to(dev), sv.to(dev) * torch.linspace(1.03, 2.33, n, device=dev)
+    x = (torch.randn(B, n, generator=torch.Generator().manual_seed(B)).clamp_(-2, 2) * size).to(dev).to(dtype)
+    y = forward_packed(x, packed, su, sv, 1.0, 0.0, 0.0135, out_dtype=torch.float32)
+    W = _decode(codes.to(dev).unsqueeze(0), [0], [1.0]).reshape(m, n).double()
+    want = structured_T(structured_T(x.double() * sv.double()) @ W.T * 0.0135) * su.double()
+    # the fp16 operand's 2.2e-4 of a row's norm; one 16-bit plane of bf16 products would leave 2e-3
+    rel = ((y.double() - want).norm(dim=1) / want.norm(dim=1)).max().item()
+    assert rel < 1e-3, rel
