@@ -42,22 +42,34 @@ def _two_sided(X: Tensor, left: Tensor, right: Tensor) -> Tensor:
     return out
 
 
+def _kernel_signs(t: Tensor, n: int, X: Tensor) -> bool:
+    """Whether a kernel may multiply by t in torch's place: fp32 values, one per
+    row or column, as they lie in memory, and nothing that torch would record or
+    batch (gradients, tangents, functorch's wrappers, tensor subclasses)."""
+    return (type(t) in (Tensor, torch.nn.Parameter) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and t.dtype == torch.float32 and t.shape == (n,) and t.device == X.device
+            and not t.is_neg() and not (t.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
+
+
 def _two_sided_inverse(X: Tensor, left: Tensor, right: Tensor) -> Tensor:
     """(T_m X T_n) (.) left[:, None] (.) right[None, :] (quipsharp/incoherence.py:74-83).
-    The row signs are applied before T_n, which they pass through unchanged."""
-    _lib.require_gpu(X, left, right, what="incoherence processing")
+    In the kernels the row signs are applied before T_n, which they pass through
+    unchanged."""
+    _lib.require_gpu(X, what="incoherence processing")
     X = X.float().contiguous()
     m, n = X.shape
-    left, right = left.float().expand(m).contiguous(), right.float().expand(n).contiguous()
     fm, fn = kron_factor(m), kron_factor(n)
     Km = hartley_matrix(fm[0], X.device) if fm[0] > 1 else None
     Kn = hartley_matrix(fn[0], X.device) if fn[0] > 1 else None
     L = _lib.lib()
     s = _lib.stream_of(X)
     out = torch.empty_like(X)
-    _lib.check(L.qs_rht_f32(_lib.ptr(X), _lib.ptr(out), 1, m, n, None, None, _lib.ptr(left), fm[0], _lib.ptr(Km), s))
-    _lib.check(L.qs_rht_f32(_lib.ptr(out), _lib.ptr(out), m, n, 1, None, None, _lib.ptr(right), fn[0], _lib.ptr(Kn), s))
-    return out
+    fused = _kernel_signs(left, m, X) and _kernel_signs(right, n, X)
+    row, col = (left.contiguous(), right.contiguous()) if fused else (None, None)
+    _lib.check(L.qs_rht_f32(_lib.ptr(X), _lib.ptr(out), 1, m, n, None, None, _lib.ptr(row), fm[0], _lib.ptr(Km), s))
+    _lib.check(L.qs_rht_f32(_lib.ptr(out), _lib.ptr(out), m, n, 1, None, None, _lib.ptr(col), fn[0], _lib.ptr(Kn), s))
+    return out if fused else out * left.unsqueeze(1) * right.unsqueeze(0)
 
 
 def _rows(x: Tensor, pre: Tensor = None, post: Tensor = None) -> Tensor:
