@@ -127,9 +127,9 @@ int launch_bx_big(const BatchedPass& P, hipStream_t stream);
 int launch_by_big(const BatchedPass* P, int count, hipStream_t stream);
 
 // Transforms of a long batch (qs_linear_rows.hip), one row per wave: the input
-// side from kRowsInMin rows and for every length on the chunk scheme up to 32768
-// (each row and its signs on 16 bytes), the output side from kRowsOutMin rows
-// for lengths beyond the chunk kernels' 12288.
+// side from kRowsInMin rows and for every length on the chunk scheme up to 32768,
+// 16384 for fp32 rows (each row and its signs on 16 bytes), the output side from
+// kRowsOutMin rows for lengths beyond the chunk kernels' 12288.
 constexpr int64_t kRowsInMin = 160, kRowsOutMin = 320;
 bool rows_input_fits(const BatchedPass& P);
 bool rows_output_fits(const BatchedPass& P);

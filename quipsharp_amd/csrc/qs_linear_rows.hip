@@ -47,6 +47,11 @@ namespace {
 constexpr int kRowsThreads = 256;
 constexpr int kRowsWaves = kRowsThreads / 64;  // rows per tile
 constexpr int kRowsMaxS = 128;
+// Longest fp32 rows.  Beyond them shorter batches run xin_kernel, which is fp32
+// throughout: error against 64 bits at 160 rows of 18944 2.082e-4 there, 2.091e-4
+// with two bf16 planes here (25600: 2.084e-4 and 2.097e-4).  fp16 rows, whose M is
+// two fp16 planes, have xin_kernel's error at every length (18944: 2.080e-4 both).
+constexpr int64_t kRowsMaxFp32 = 16384;
 constexpr int kRowsMStr = kRowsMaxS + 8;  // 16-bit words per row of M in LDS
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -660,6 +665,7 @@ bool rows_transform_fits(int64_t len, int p) {
 }
 bool rows_input_fits(const BatchedPass& P) {
   const size_t es = P.x_dtype == QS_DTYPE_F32 ? 4 : 2;
+  if (P.x_dtype == QS_DTYPE_F32 && P.n > kRowsMaxFp32) return false;
   return P.frag && P.B >= kRowsInMin && rows_transform_fits(P.n, P.pn) && (reinterpret_cast<uintptr_t>(P.x) & 15) == 0 &&
          P.ldx * es % 16 == 0 && (reinterpret_cast<uintptr_t>(P.sv) & (P.sbits ? 3 : 15)) == 0;
 }

@@ -154,3 +154,13 @@ def test_input_factors_that_are_not_signs(dev, n, B, dtype, size):
     # the fp16 operand's 2.2e-4 of a row's norm; one 16-bit plane of bf16 products would leave 2e-3
     rel = ((y.double() - want).norm(dim=1) / want.norm(dim=1)).max().item()
     assert rel < 1e-3, rel
+
+
+@pytest.mark.parametrize("n", [17408, 18944, 25600, 32768])
+def test_long_fp32_rows_are_transformed_in_fp32(dev, n):
+    """fp32 activations beyond 16384 columns: a long batch's rows are those of a shorter one."""
+    from quipsharp_amd.quantize import forward_packed
+    packed, su, sv, _, _ = layer(dev, 256, n, n, False)
+    args = (packed, su.to(dev), sv.to(dev), 1.0, 0.0, 0.0135)
+    x = torch.randn(160, n, generator=torch.Generator().manual_seed(n)).to(dev)
+    assert torch.equal(forward_packed(x, *args)[:159], forward_packed(x[:159].contiguous(), *args))
