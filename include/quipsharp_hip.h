@@ -171,7 +171,8 @@ int qs_rht_f32(const float *in, float *out, int64_t outer, int64_t n, int64_t in
 int qs_pack_codes(const void *codes, int code_bytes, int64_t m, int64_t n, int stage_kind,
                   int layout, void *out, qs_stream_t stream);
 
-/* Workspace bytes needed by qs_linear_forward for this shape and batch. */
+/* Workspace bytes that serve qs_linear_forward for this shape and every batch
+ * up to this one (they never fall as the batch grows). */
 size_t qs_linear_workspace_bytes(int64_t m, int64_t n, int64_t batch, int layout);
 
 /* y = su (.) T_m( layer_scale * W_hat @ T_n(sv (.) x) ) + bias for batch rows,
@@ -205,9 +206,10 @@ int qs_linear_forward(const void *x, int x_dtype, int64_t ldx, int64_t batch, in
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
  * The workspace is a device array in the library's code object, one copy of
  * QS_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; this entry
- * point calls no hipMalloc / hipFree.  Shapes whose workspace
- * (qs_linear_workspace_bytes) exceeds it return QS_ERR_UNSUPPORTED before
- * anything is launched.  Every shape with m, n <= 32768 fits at 1..128 rows;
+ * point calls no hipMalloc / hipFree.  Calls that need more than it return
+ * QS_ERR_UNSUPPORTED before anything is launched; none does for which
+ * qs_linear_workspace_bytes gives at most its size.  Every shape with m, n <=
+ * 32768 fits at 1..128 rows;
  * wide prefill batches (256 rows and more) of most shapes do not (11008 x
  * 4096 at 4096 rows needs 219 MB).  Every call on one GPU shares that
  * GPU's array: calls that may overlap on one GPU (other streams, other host
@@ -246,7 +248,8 @@ typedef struct qs_linear_job {
   int sign_bits;        /* nonzero: su and sv are packed sign bits (see QS_SIGNS_BITS); the same for every job */
 } qs_linear_job;
 
-/* Workspace bytes for qs_linear_forward_group: ms[count] output sizes. */
+/* Workspace bytes for qs_linear_forward_group: ms[count] output sizes, every
+ * batch up to this one. */
 size_t qs_linear_group_workspace_bytes(int64_t n, int64_t batch, int count, const int64_t *ms);
 
 /* Several linears that read the same input x in one launch: for each job,

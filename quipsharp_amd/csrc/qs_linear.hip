@@ -116,8 +116,9 @@ WsLayout ws_layout(int64_t m, int64_t n, int64_t batch, int layout) {
   if (L.wide) {
     // partial groups of the wide GEMM, or the 16-row passes of the
     // decode-matvec (which also takes this layout)
-    const size_t a = wide_partial_bytes(m, n, B, cu_count()), b = (size_t)L.SG * kMaxTileBatch * m * 4;
-    L.y1p = off; off = align256(off + (a > b ? a : b));
+    const int g0 = wide_splits(m, n, B, cu_count(), false), g1 = wide_splits(m, n, B, cu_count(), true);
+    const size_t a = (size_t)(g0 > g1 ? g0 : g1) * B, b = (size_t)L.SG * kMaxTileBatch;
+    L.y1p = off; off = align256(off + (a > b ? a : b) * m * 4);
   } else {
     const int sgp = L.SG > L.fused.SG ? L.SG : L.fused.SG;
     L.y1p = off; off = align256(off + (size_t)sgp * B * m * 4);
@@ -131,6 +132,19 @@ WsLayout ws_layout(int64_t m, int64_t n, int64_t batch, int layout) {
   }
   L.total = off;
   return L;
+}
+
+// Bytes of a workspace for every call of up to `batch` rows: the largest of
+// their layouts' totals, each of which is all that its own call asks for.
+// Only the partial sums of the wide GEMM, a layout's last region, can shrink as
+// the rows grow (fewer slice groups), and the step from 16 rows to 17.
+size_t ws_bytes(int64_t m, int64_t n, int64_t batch, int layout) {
+  const WsLayout W = ws_layout(m, n, batch, layout);
+  if (!W.wide) return W.total;
+  const size_t wide = align256(W.y1p + wide_partial_bytes(m, n, batch, cu_count()));
+  const size_t narrow = ws_layout(m, n, kMaxTileBatch, layout).total;
+  const size_t most = wide > narrow ? wide : narrow;
+  return most > W.total ? most : W.total;
 }
 
 
@@ -890,7 +904,7 @@ extern "C" int qs_busy_wait(int64_t nanoseconds, qs_stream_t stream) {
 
 extern "C" size_t qs_linear_workspace_bytes(int64_t m, int64_t n, int64_t batch, int layout) {
   if (m <= 0 || n <= 0 || batch <= 0) return 0;
-  return ws_layout(m, n, batch, layout).total;
+  return ws_bytes(m, n, batch, layout);
 }
 
 extern "C" int qs_linear_forward(const void* x, int x_dtype, int64_t ldx, int64_t batch, int64_t n, int64_t m,
@@ -1209,7 +1223,7 @@ extern "C" size_t qs_linear_group_workspace_bytes(int64_t n, int64_t batch, int 
   for (int g = 0; g < count; ++g)
     if (ms[g] <= 0) return 0;
   size_t total = group_prefix_bytes(count, n, [&](int g) { return ms[g]; });
-  for (int g = 0; g < count; ++g) total += ws_layout(ms[g], n, batch, QS_LAYOUT_TILED).total;
+  for (int g = 0; g < count; ++g) total += ws_bytes(ms[g], n, batch, QS_LAYOUT_TILED);
   return total;
 }
 

@@ -179,9 +179,8 @@ struct WideMfma {
 // limit.  Up to 128 rows two work-groups per CU, which run side by side and
 // cover each other's loads, while the partial sums take at most 8 MiB.
 int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2);
-// Bytes of partial sums that a workspace for B rows of either stage count holds:
-// up to 128 rows also those of any fewer rows, whose second work-group per CU
-// can take more.
+// Most bytes of partial sums of any wide call of up to B rows, of either stage
+// count (fewer rows can have more groups, and more bytes).
 size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu);
 // Linears of one shape (m, n, B) with one stage above 128 rows whose tiles
 // together fit one round over the CUs share one producer / consumer GEMM

@@ -559,14 +559,16 @@ int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
 }
 
 size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu) {
-  size_t most = 0;
-  for (int has2 = 0; has2 < 2; ++has2) {
-    size_t b = (size_t)wide_splits(m, n, B, ncu, has2) * B * m * 4;
-    most = b > most ? b : most;
-    if (B > 16 * kWgMaxCols) continue;
-    b = (size_t)groups_within(wide_tiles(m, B, has2), n, 2 * ncu) * B * m * 4;
-    b = b < (size_t)kWgPartialBytes ? b : (size_t)kWgPartialBytes;
-    most = b > most ? b : most;
+  const int64_t row = m * 4, nrt = wide_tiles(m, 1, false), first = B < 16 * kWgMaxCols ? B : 16 * kWgMaxCols;
+  // up to 128 rows: one column of tiles, whatever the rows
+  size_t most = (size_t)(groups_within(nrt, n, ncu) * first * row), two = (size_t)(groups_within(nrt, n, 2 * ncu) * first * row);
+  if (two > (size_t)kWgPartialBytes) two = (size_t)kWgPartialBytes;
+  if (two > most) most = two;
+  // beyond: the most rows of each count of groups (a second stage never has more groups than one stage)
+  for (int64_t g = 1; g <= kWideMaxGroups && g <= n / 256 && B > first; ++g) {
+    const int64_t rows = g == 1 ? B : ncu / (g * nrt) * 256;
+    const size_t b = (size_t)(g * (rows < B ? rows : B) * row);
+    if (rows > first && b > most) most = b;
   }
   return most;
 }

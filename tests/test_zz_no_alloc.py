@@ -117,3 +117,21 @@ def test_noalloc_rejects_oversized(dev, m, n, rows):
     torch.cuda.synchronize()
     assert bool((y == 7.0).all())
     assert np.isfinite(need)
+
+
+def test_bytes_of_a_call_and_of_every_smaller_one(dev):
+    """One workspace sized for 300 rows serves 256 (whose GEMM has more slice
+    groups and more partial sums), 100 and 16 rows; the allocation-free forward
+    asks for the call's own bytes (300 rows fit where 256 do not)."""
+    from quipsharp_amd import _lib
+    lib = _lib.lib()
+    L = _linear(dev, 4096, 4096, 3, True, False)
+    ws = torch.zeros(lib.qs_linear_workspace_bytes(4096, 4096, 300, L["packed"].layout), dtype=torch.uint8, device=dev)
+    x = torch.randn(300, 4096, generator=torch.Generator().manual_seed(2)).to(dev).bfloat16()
+    for rows in (256, 100, 300, 16):
+        y = torch.empty(rows, 4096, dtype=torch.bfloat16, device=dev)
+        _lib.check(lib.qs_linear_forward(*_args(L, x[:rows], y), _lib.ptr(ws), ws.numel(), None, None, _lib.stream_of(x)))
+        assert torch.equal(y, _with_workspace(L, x[:rows]))
+    assert torch.equal(_noalloc(L, x), _with_workspace(L, x))
+    y = torch.empty(256, 4096, dtype=torch.bfloat16, device=dev)
+    assert lib.qs_linear_forward_noalloc(*_args(L, x[:256], y), _lib.stream_of(x)) == 3
