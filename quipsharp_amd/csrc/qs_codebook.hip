@@ -563,8 +563,11 @@ struct ChunkLds {
   float dinv[kChunkBlocks * 64];
 };
 constexpr size_t chunk_lds(int rows) { return sizeof(ChunkLds) + (size_t)rows * 3 * kChunkLd * sizeof(float); }
+constexpr int kChunkMaxRows = 32;  // of a work-group
+constexpr int kChunkMaxLds = (int)chunk_lds(kChunkMaxRows);
+static_assert(kChunkMaxLds <= 160 * 1024, "LDS budget");
 
-__global__ __launch_bounds__(512) void ldlq_chunk_kernel(ChunkArgs A) {
+__global__ __launch_bounds__(16 * kChunkMaxRows) void ldlq_chunk_kernel(ChunkArgs A) {
   extern __shared__ char sm[];
   ChunkLds& S = *reinterpret_cast<ChunkLds*>(sm);
   float* rows = reinterpret_cast<float*>(sm + sizeof(ChunkLds));  // per row: p (then codes), w (then E), wq
@@ -942,9 +945,10 @@ extern "C" int qs_ldlq_chunk(const float* w, int64_t ldw, float* wq, int64_t ldw
   A.code_stride = code_stride;
   // 16 rows per work-group (one per CU by its LDS) up to one round of the 256
   // CUs, 32 beyond: two waves per SIMD then share H's chunk
-  const int rows = m > 16 * 256 ? 32 : 16;
+  const int rows = m > 16 * 256 ? kChunkMaxRows : 16;
   const size_t lds = chunk_lds(rows);
-  QS_HIP(hipFuncSetAttribute((const void*)ldlq_chunk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // the limit is the same for every call, so that threads do not lower each other's
+  QS_HIP(hipFuncSetAttribute((const void*)ldlq_chunk_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kChunkMaxLds));
   hipLaunchKernelGGL(ldlq_chunk_kernel, dim3((unsigned)((m + rows - 1) / rows)), dim3(16 * rows), lds,
                      as_stream(stream), A);
   QS_LAUNCHED("ldlq_chunk_kernel");

@@ -480,7 +480,8 @@ struct WyLds {
 constexpr size_t wy_lds(int groups) {
   return sizeof(WyLds) - (size_t)(kMaxGroups16 - groups) * 2 * 16 * kRowsMStr * sizeof(uint16_t);
 }
-static_assert(wy_lds(kMaxGroups16) <= 160 * 1024, "LDS budget");
+constexpr int kWyMaxLds = (int)wy_lds(kMaxGroups16);
+static_assert(kWyMaxLds <= 160 * 1024, "LDS budget");
 
 // LO: a job's M has a second plane.
 template <bool SB, bool LO>
@@ -756,7 +757,8 @@ int launch_wy(const BatchedPass* P, int count, hipStream_t stream) {
   }
   const size_t lds = wy_lds(most);
   auto launch = [&](auto kernel) {
-    QS_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    // the most that any call takes: a limit of its own could be another thread's next launch's
+    QS_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kWyMaxLds));
     hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(kWyThreads), lds, stream, A);
     return (int)QS_OK;
   };

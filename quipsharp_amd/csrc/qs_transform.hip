@@ -17,6 +17,7 @@ namespace qs {
 namespace {
 
 constexpr int kMaxRowLen = 32768;  // 128 KiB of LDS
+constexpr int kMaxRowLds = padded_len(kMaxRowLen) * 4;
 constexpr int kSpan = 4096;        // elements per work-group when rows are shorter
 constexpr int kKronTile = 8;       // outputs per LDS read of the odd-factor stage
 
@@ -316,9 +317,9 @@ void launch_cols(const ColArgs& A, int64_t groups, hipStream_t s) {
 
 template <int BITS>
 int launch_rows(const RowArgs& A, const float* K, int64_t blocks, int threads, size_t lds, hipStream_t s) {
-  if (lds > 65536)
+  if (lds > 65536)  // the longest row's: a limit of its own could be another thread's next launch's
     QS_HIP(hipFuncSetAttribute((const void*)rht_rows_kernel<BITS>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)lds));
+                               kMaxRowLds));
   hipLaunchKernelGGL(rht_rows_kernel<BITS>, dim3((unsigned)blocks), dim3(threads), lds, s, A, K);
   QS_LAUNCHED("rht_rows_kernel");
   return QS_OK;
