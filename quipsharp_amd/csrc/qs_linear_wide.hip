@@ -266,6 +266,13 @@ __global__ __launch_bounds__(kWgThreads, 2) void wg_kernel(WgArgs A) {
 
 template <bool HAS2, int NB, int WC>
 int launch_wg(const WgArgs& A, unsigned grid, hipStream_t stream) {
+  static int done = 0;
+  if (!done) {
+    hipFuncAttributes fa{};
+    QS_HIP(hipFuncGetAttributes(&fa, (const void*)wg_kernel<HAS2, NB, WC>));
+    QS_REQUIRE(fa.sharedSizeBytes == 0, "wg_kernel: static LDS would move the tables off address 0");
+    done = 1;
+  }
   hipLaunchKernelGGL((wg_kernel<HAS2, NB, WC>), dim3(grid), dim3(kWgThreads), kWgLds, stream, A);
   QS_LAUNCHED("wg_kernel");
   return QS_OK;
