@@ -76,7 +76,7 @@ struct WpJob {
   const _Float16* sgf;
   float s1;
   int m, RB, nrt, SGk, spg;
-  int t0;              // first tile of the launch
+  int wg0, tiles;      // first work-group (a multiple of 8), tiles
 };
 
 struct WgArgs {
@@ -84,7 +84,6 @@ struct WgArgs {
   int nrt, nct;        // work-group tiles along the weight rows / activation rows
   int SGk, spg;        // slice groups, slices per group
   int njobs;
-  int tiles;           // wg_kernel: of all jobs
   WpJob job[QS_MAX_GROUP];
 };
 
@@ -99,20 +98,22 @@ __global__ __launch_bounds__(kWgThreads, 2) void wg_kernel(WgArgs A) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q = lane >> 4, r16 = lane & 15;
 
-  // Tiles are ordered weight-row tiles fastest, then activation tiles, then
-  // slice groups, then jobs, and dealt to the XCDs in contiguous runs:
-  // work-group i runs on XCD i % 8, so tile (i % 8) * ceil(T / 8) + i / 8 keeps
-  // each XCD's L2 on a few activation columns and slice groups (the grid is
-  // rounded up to a multiple of 8; the surplus work-groups exit at once).
-  const int per = (A.tiles + 7) >> 3;
-  int bid = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-  if (bid >= A.tiles) return;
+  // A job's tiles are ordered weight-row tiles fastest, then activation tiles,
+  // then slice groups, and dealt to the XCDs in contiguous runs: work-group i
+  // runs on XCD i % 8, so tile (i % 8) * ceil(T / 8) + i / 8 keeps each XCD's L2
+  // on a few activation columns and slice groups (surplus work-groups exit at
+  // once).  Each job by itself: in one run over the jobs the tiles of a large
+  // linear, which has few slice groups of many slices, fell on a few XCDs (two
+  // stages, 5120 columns to 8192 + 1024 + 1024 at 300 rows: 285 us in one run,
+  // 220 in a launch each, 162 dealt job by job; linears of one shape equal).
   int jj = 0;
 #pragma unroll
   for (int k = 1; k < QS_MAX_GROUP; ++k)
-    if (k < A.njobs && bid >= A.job[k].t0) jj = k;
+    if (k < A.njobs && (int)blockIdx.x >= A.job[k].wg0) jj = k;
   const WpJob& J = A.job[jj];
-  bid -= J.t0;
+  const int local = (int)blockIdx.x - J.wg0;
+  int bid = (local & 7) * ((J.tiles + 7) >> 3) + (local >> 3);
+  if (bid >= J.tiles) return;
   const int rt = bid % J.nrt;
   bid /= J.nrt;
   const int ct = bid % A.nct;
@@ -587,7 +588,7 @@ int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu) {
 }
 
 namespace {
-int wide_args(const WideMfma* G, int count, WgArgs& A) {
+int wide_args(const WideMfma* G, int count, WgArgs& A, int64_t& wgs) {
   const bool has2 = G[0].codes1 != nullptr;
   const int cols = use_wp(G[0].B, has2) ? 256 : 16 * wg_cols(G[0].B);
   A.m = (int)G[0].m;
@@ -599,7 +600,7 @@ int wide_args(const WideMfma* G, int count, WgArgs& A) {
   A.SGk = G[0].SGk;
   A.spg = (A.S + A.SGk - 1) / A.SGk;
   A.njobs = count;
-  int64_t tiles = 0;
+  wgs = 0;
   for (int j = 0; j < count; ++j) {
     const WideMfma& F = G[j];
     QS_REQUIRE(F.m % 16 == 0 && F.n % 256 == 0 && F.B >= 1, "wide GEMM: m %% 16, n %% 256");
@@ -607,12 +608,12 @@ int wide_args(const WideMfma* G, int count, WgArgs& A) {
     QS_REQUIRE(F.m * F.n / 4 < ((int64_t)1 << 40), "wide GEMM: codes too large");
     QS_REQUIRE(F.n == G[0].n && F.B == A.B && (F.codes1 != nullptr) == has2, "wide GEMM: linears of one operand width");
     const int RB = (int)(F.m / 16), nrt = (RB + kWgRowTiles - 1) / kWgRowTiles;
+    const int64_t tiles = (int64_t)nrt * A.nct * F.SGk;
     A.job[j] = WpJob{static_cast<const uint16_t*>(F.codes0), F.x2f, F.y1p, F.s0, static_cast<const uint8_t*>(F.codes1),
-                     F.sgf, F.s1, (int)F.m, RB, nrt, F.SGk, (A.S + F.SGk - 1) / F.SGk, (int)tiles};
-    tiles += (int64_t)nrt * A.nct * F.SGk;
-    QS_REQUIRE(tiles < ((int64_t)1 << 30), "wide GEMM: grid too large");
+                     F.sgf, F.s1, (int)F.m, RB, nrt, F.SGk, (A.S + F.SGk - 1) / F.SGk, (int)wgs, (int)tiles};
+    wgs += (tiles + 7) / 8 * 8;
+    QS_REQUIRE(wgs < ((int64_t)1 << 30), "wide GEMM: grid too large");
   }
-  A.tiles = (int)tiles;
   return QS_OK;
 }
 }  // namespace
@@ -620,15 +621,18 @@ int wide_args(const WideMfma* G, int count, WgArgs& A) {
 int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream) {
   QS_REQUIRE(count >= 1 && count <= QS_MAX_GROUP, "wide GEMM: 1..%d linears", QS_MAX_GROUP);
   WgArgs A{};
-  const int rc = wide_args(G, count, A);
+  int64_t wgs = 0;
+  const int rc = wide_args(G, count, A, wgs);
   if (rc) return rc;
-  const unsigned grid = (unsigned)((A.tiles + 7) / 8 * 8);  // XCD-contiguous tile order (see wg_kernel)
   const bool has2 = G[0].codes1 != nullptr;
   if (use_wp(A.B, has2)) {
     for (int j = 1; j < count; ++j)
       QS_REQUIRE(G[j].m == G[0].m && G[j].SGk == G[0].SGk, "wide GEMM: one shape beyond %d rows", 16 * kWgMaxCols);
-    return launch_wp(A, grid, stream);
+    // one run of tiles over the jobs, which are alike
+    const int64_t tiles = (int64_t)count * A.job[0].tiles;
+    return launch_wp(A, (unsigned)((tiles + 7) / 8 * 8), stream);
   }
+  const unsigned grid = (unsigned)wgs;
   return has2 ? launch_wg<true>(A, wg_cols(A.B), grid, stream) : launch_wg<false>(A, wg_cols(A.B), grid, stream);
 }
 
