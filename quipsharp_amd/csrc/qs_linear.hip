@@ -1150,10 +1150,6 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
     bool one_shape = true;
     for (int g = 0; g < count; ++g) one_shape = one_shape && P[g].m == P[0].m && P[g].codes1 == nullptr;
     const int gsk = one_shape ? wide_group_splits(P[0].m, n, batch, count, cu_count()) : 0;
-    bool shared = true;
-    for (int g = 0; g < count; ++g)
-      shared = shared && (P[g].codes1 != nullptr) == (P[0].codes1 != nullptr) &&
-               wide_shares_launch(batch, P[g].codes1 != nullptr);
     WideMfma F[QS_MAX_GROUP];
     for (int g = 0; g < count; ++g) {
       F[g] = WideMfma{};
@@ -1168,14 +1164,16 @@ static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t b
       F[g].sgf = P[g].sg;
       F[g].y1p = P[g].y1p;
       F[g].SGk = gsk ? gsk : wide_splits(P[g].m, n, batch, cu_count(), P[g].codes1 != nullptr);
-      if (!gsk && !shared) {
-        rc = launch_linear_wide(&F[g], 1, s);
-        if (rc) return rc;
-      }
       P[g].SG = F[g].SGk;  // partial groups summed by the output kernels
     }
-    if (gsk || shared) {
-      rc = launch_linear_wide(F, count, s);
+    bool done[QS_MAX_GROUP] = {};
+    for (int g = 0; g < count; ++g) {
+      if (done[g]) continue;
+      WideMfma L[QS_MAX_GROUP];
+      int nl = 0;
+      for (int h = g; h < count; ++h)
+        if (!done[h] && (h == g || gsk || wide_shares_launch(F[g], F[h]))) L[nl++] = F[h], done[h] = true;
+      rc = launch_linear_wide(L, nl, s);
       if (rc) return rc;
     }
     if (mv_end) QS_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(mv_end), s));

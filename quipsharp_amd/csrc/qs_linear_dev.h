@@ -189,10 +189,11 @@ size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu);
 // separate calls up to the fp32 summation order).  Returns those slice
 // groups, or 0 when the linears take one launch each.
 int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu);
-// Whether linears of B rows of one operand width share a launch whatever their
-// m, each with its own slice groups (the decode-in-the-loop kernel), or only
-// those of one shape by wide_group_splits (the producer / consumer kernel).
-bool wide_shares_launch(int64_t B, bool has2);
+// Whether two linears of one operand width, row count and stage count share a
+// launch, each with its own slice groups: those of the decode-in-the-loop
+// kernel, and up to 128 rows those of one m of the producer / consumer kernel
+// (beyond, only by wide_group_splits).
+bool wide_shares_launch(const WideMfma& a, const WideMfma& b);
 int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream);
 
 

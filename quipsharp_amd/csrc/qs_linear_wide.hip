@@ -6,11 +6,13 @@
 // its K loop (byte LUTs in LDS, exactly as the narrow kernels) and feeds
 // every decoded fragment to several 16 x 16 x 32 fp16 MFMAs; the codes' +-1/4
 // shifts are one extra MFMA per slice against the operand's group sums.
-// Single-stage calls of more than 128 rows take wp_kernel instead, which
-// splits decoding and multiplying between the waves of a work-group.  The
-// input and output transforms around it are the per-row kernels of the
-// batched path (qs_linear_batched.hip) or, outside the chunk scheme, the
-// LDS-radix kernels of qs_linear.hip, writing the fragment-major operand.
+// Single-stage calls of more than 128 rows, and large linears from 65, take
+// wp_kernel instead, which splits decoding and multiplying between the waves of
+// a work-group.  The transforms around it write the fragment-major operand and
+// read the partial sums: one row per wave for a long batch (qs_linear_rows.hip),
+// otherwise the per-row kernels of the batched path (qs_linear_batched.hip,
+// qs_linear_big.hip) or, for lengths that these do not cover, the LDS-radix
+// kernels of qs_linear.hip.
 #include <type_traits>
 
 #include "qs_forward_dev.h"
@@ -31,16 +33,18 @@ constexpr int kDqOffLut1 = 32768;          // 256 x uint4 (E8 1-bit rows, fp16)
 // a second stage: 10 and 26 clocks per 64 codes) and the operand through the
 // L1 (1 KiB a fragment, 16 clocks).  With WC = 1 every wave has two 16-row code
 // tiles of its own and multiplies all of the activation rows, so that a code is
-// decoded once and a fragment read four times; with WC = 2, beyond 64 rows of
-// one stage, the waves are 2 x 2, four code tiles by half the rows each, both
-// twice.  (A wave with all the weight rows and activation rows of its own, as
-// this kernel was, decodes every code four times.)  A wave's code tiles go from
-// memory to its registers a slice ahead, and the loop has no barrier.
+// decoded once and a fragment read four times; with WC = 2, 65 to 128 rows of
+// one stage (the large linears of which wp_kernel takes), the waves are 2 x 2,
+// four code tiles by half the rows each, both twice.  (A wave with all the weight
+// rows and activation rows of its own, as this kernel was, decodes every code
+// four times.)  A wave's code tiles go from memory to its registers a slice
+// ahead, and the loop has no barrier.
 //
 // A layer's linears and transforms, graph-replayed (that form -> now):
 //   Llama-3-8B 3 bits  17 rows 178 -> 127 us, 45 202 -> 163, 128 308 -> 267, 700 1256 -> 1154
 //   Qwen3-32B 2 bits   17 rows 250 -> 184 us, 45 291 -> 239, 64 325 -> 272
-//   the same, 128 rows 437 -> 417 us (WC = 1: 520); 3 bits 559 -> 501 (WC = 2: 522)
+//   the same, 128 rows 437 -> 417 us (WC = 1: 520), 359 with wp_kernel for the
+//   large ones; 3 bits 559 -> 501 (WC = 2: 522)
 //
 // Linears of one operand width share a launch, each with the slice groups that
 // it has alone, so that the outputs do not depend on the company.
@@ -59,9 +63,19 @@ inline int wg_cols(int64_t B) {
   const int64_t nb = (nbt + nct - 1) / nct;
   return nb <= 2 ? 2 : nb <= 3 ? 3 : nb <= 4 ? 4 : nb <= 6 ? 6 : 8;
 }
-// Single-stage calls of more than 128 rows run wp_kernel (256 activation rows
-// per work-group).
-inline bool use_wp(int64_t B, bool has2) { return !has2 && B > 16 * kWgMaxCols; }
+// Single-stage linears run wp_kernel (256 activation rows per work-group) beyond
+// 128 rows, those of more than 2^24 weights beyond 64: wg_kernel's 2 x 2 form
+// wants two work-groups per CU, which one linear of 65 to 128 rows seldom has
+// (alone it was 2 to 22 % slower than the form before it).
+// One linear, 128 rows, wg_kernel -> wp_kernel: 5120 x 25600 123 -> 89 us, 11008
+// x 4096 56.2 -> 45.6, 4096 x 4096 34.2 -> 33.1.  The smaller ones are mostly
+// members of a group, whose launch wg_kernel shares whatever their m: 4096 to
+// 4096 + 1024 + 1024 42.5 us, by wp_kernel, each or together, 46.6 and more.
+constexpr int64_t kWpWeights = 1 << 24;
+inline bool use_wp(int64_t m, int64_t n, int64_t B, bool has2) {
+  return !has2 && (B > 16 * kWgMaxCols || (B > 64 && m * n > kWpWeights));
+}
+inline bool use_wp(const WideMfma& F) { return use_wp(F.m, F.n, F.B, F.codes1 != nullptr); }
 
 // One linear of a launch.  wp_kernel: linears of one shape (m, n, rows) that
 // read their own operands share a launch, job j taking tiles j T1 .. (j + 1) T1
@@ -290,7 +304,7 @@ int launch_wg(const WgArgs& A, int cols, unsigned grid, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// Producer / consumer variant for long single-stage batches
+// Producer / consumer variant for single-stage batches (use_wp)
 // ---------------------------------------------------------------------------
 // The wave that feeds the matrix cores should issue nothing but MFMAs and
 // their operand loads: VALU work issued by that wave is not hidden behind its
@@ -544,8 +558,8 @@ int launch_wp(const WgArgs& A, unsigned grid, hipStream_t stream) {
 }  // namespace
 
 // Work-group tiles of one linear (128 weight rows by the work-group's activation rows).
-static int64_t wide_tiles(int64_t m, int64_t B, bool has2) {
-  const int64_t cols = use_wp(B, has2) ? 256 : 16 * wg_cols(B);
+static int64_t wide_tiles(int64_t m, int64_t n, int64_t B, bool has2) {
+  const int64_t cols = use_wp(m, n, B, has2) ? 256 : 16 * wg_cols(B);
   return ((m / 16 + kWgRowTiles - 1) / kWgRowTiles) * ((B + cols - 1) / cols);
 }
 static int groups_within(int64_t tiles, int64_t n, int64_t limit) {
@@ -556,10 +570,10 @@ static int groups_within(int64_t tiles, int64_t n, int64_t limit) {
 }
 
 int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
-  const int64_t tiles = wide_tiles(m, B, has2);
+  const int64_t tiles = wide_tiles(m, n, B, has2);
   int g = groups_within(tiles, n, ncu);
   // up to 128 rows a second work-group per CU, while the partial sums stay few
-  if (B <= 16 * kWgMaxCols) {
+  if (B <= 16 * kWgMaxCols && !use_wp(m, n, B, has2)) {
     const int g2 = groups_within(tiles, n, 2 * ncu), most = (int)(kWgPartialBytes / (B * m * 4));
     if (g2 > g && most > g) g = g2 < most ? g2 : most;
   }
@@ -567,7 +581,7 @@ int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
 }
 
 size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu) {
-  const int64_t row = m * 4, nrt = wide_tiles(m, 1, false), first = B < 16 * kWgMaxCols ? B : 16 * kWgMaxCols;
+  const int64_t row = m * 4, nrt = wide_tiles(m, n, 1, false), first = B < 16 * kWgMaxCols ? B : 16 * kWgMaxCols;
   // up to 128 rows: one column of tiles, whatever the rows
   size_t most = (size_t)(groups_within(nrt, n, ncu) * first * row), two = (size_t)(groups_within(nrt, n, 2 * ncu) * first * row);
   if (two > (size_t)kWgPartialBytes) two = (size_t)kWgPartialBytes;
@@ -582,15 +596,15 @@ size_t wide_partial_bytes(int64_t m, int64_t n, int64_t B, int ncu) {
 }
 
 int wide_group_splits(int64_t m, int64_t n, int64_t B, int count, int ncu) {
-  if (count < 2 || !use_wp(B, false)) return 0;
-  const int64_t tiles = wide_tiles(m, B, false) * count;
+  if (count < 2 || B <= 16 * kWgMaxCols) return 0;
+  const int64_t tiles = wide_tiles(m, n, B, false) * count;
   return tiles > ncu ? 0 : groups_within(tiles, n, ncu);
 }
 
 namespace {
 int wide_args(const WideMfma* G, int count, WgArgs& A, int64_t& wgs) {
   const bool has2 = G[0].codes1 != nullptr;
-  const int cols = use_wp(G[0].B, has2) ? 256 : 16 * wg_cols(G[0].B);
+  const int cols = use_wp(G[0]) ? 256 : 16 * wg_cols(G[0].B);
   A.m = (int)G[0].m;
   A.B = G[0].B;
   A.S = (int)(G[0].n / 256);
@@ -606,7 +620,8 @@ int wide_args(const WideMfma* G, int count, WgArgs& A, int64_t& wgs) {
     QS_REQUIRE(F.m % 16 == 0 && F.n % 256 == 0 && F.B >= 1, "wide GEMM: m %% 16, n %% 256");
     QS_REQUIRE(F.SGk >= 1 && F.SGk <= kWideMaxGroups, "wide GEMM: 1..%d slice groups", kWideMaxGroups);
     QS_REQUIRE(F.m * F.n / 4 < ((int64_t)1 << 40), "wide GEMM: codes too large");
-    QS_REQUIRE(F.n == G[0].n && F.B == A.B && (F.codes1 != nullptr) == has2, "wide GEMM: linears of one operand width");
+    QS_REQUIRE(F.n == G[0].n && F.B == A.B && (F.codes1 != nullptr) == has2 && use_wp(F) == use_wp(G[0]),
+               "wide GEMM: linears of one operand width and kernel");
     const int RB = (int)(F.m / 16), nrt = (RB + kWgRowTiles - 1) / kWgRowTiles;
     const int64_t tiles = (int64_t)nrt * A.nct * F.SGk;
     A.job[j] = WpJob{static_cast<const uint16_t*>(F.codes0), F.x2f, F.y1p, F.s0, static_cast<const uint8_t*>(F.codes1),
@@ -625,9 +640,9 @@ int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream) {
   const int rc = wide_args(G, count, A, wgs);
   if (rc) return rc;
   const bool has2 = G[0].codes1 != nullptr;
-  if (use_wp(A.B, has2)) {
+  if (use_wp(G[0])) {
     for (int j = 1; j < count; ++j)
-      QS_REQUIRE(G[j].m == G[0].m && G[j].SGk == G[0].SGk, "wide GEMM: one shape beyond %d rows", 16 * kWgMaxCols);
+      QS_REQUIRE(G[j].m == G[0].m && G[j].SGk == G[0].SGk, "wide GEMM: wp_kernel takes linears of one shape");
     // one run of tiles over the jobs, which are alike
     const int64_t tiles = (int64_t)count * A.job[0].tiles;
     return launch_wp(A, (unsigned)((tiles + 7) / 8 * 8), stream);
@@ -636,6 +651,9 @@ int launch_linear_wide(const WideMfma* G, int count, hipStream_t stream) {
   return has2 ? launch_wg<true>(A, wg_cols(A.B), grid, stream) : launch_wg<false>(A, wg_cols(A.B), grid, stream);
 }
 
-bool wide_shares_launch(int64_t B, bool has2) { return !use_wp(B, has2); }
+bool wide_shares_launch(const WideMfma& a, const WideMfma& b) {
+  if (use_wp(a) || use_wp(b)) return use_wp(a) && use_wp(b) && a.m == b.m && a.B <= 16 * kWgMaxCols;
+  return true;
+}
 
 }  // namespace qs

@@ -53,3 +53,37 @@ def test_linears_of_a_shared_launch_equal_their_own(dev, B, two):
     x = t(rng.standard_normal((B, n)))
     for lin, y in zip(lins, forward_packed_group(x, lins)):
         assert torch.equal(y, forward_packed(x, *lin))
+
+
+# both sides of the line between the two GEMM kernels: 2^24 weights from 65 rows on
+@pytest.mark.parametrize("m,n", [(4096, 4096), (4224, 4096), (5632, 3072), (1088, 25600)])
+@pytest.mark.parametrize("B", [64, 65, 97, 128, 129])
+def test_kernel_line_vs_dense_fp64(dev, m, n, B):
+    from test_gpu_rows import structured_T
+
+    from quipsharp_amd.codebooks.e8p import _decode
+    from quipsharp_amd.quantize import PackedCodes, forward_packed
+    g = torch.Generator().manual_seed(m + B)
+    codes = torch.randint(0, 65536, (m, n // 8), generator=g)
+    sign = lambda k: (torch.randint(0, 2, (k,), generator=g) * 2 - 1).float().to(dev)  # noqa: E731
+    su, sv = sign(m), sign(n)
+    x = torch.randn(B, n, generator=g).to(dev)
+    y = forward_packed(x, PackedCodes(codes.to(dev), m, n, [0]), su, sv, 1.0, 0.0, 0.0135)
+    W = _decode(codes.to(dev).unsqueeze(0), [0], [1.0]).reshape(m, n).double()
+    want = structured_T(structured_T(x.double() * sv.double()) @ W.T * 0.0135) * su.double()
+    rows = (y.double() - want).norm(dim=1) / want.norm(dim=1)
+    assert rows.max() < REL_TOL, (int(rows.argmax()), rows.max().item())
+
+
+@pytest.mark.parametrize("B", [65, 128])
+def test_group_on_both_sides_of_the_line_equals_single_calls(dev, B):
+    from quipsharp_amd.quantize import PackedCodes, forward_packed, forward_packed_group
+    n, g = 4096, torch.Generator().manual_seed(B)
+    sign = lambda k: (torch.randint(0, 2, (k,), generator=g) * 2 - 1).float().to(dev)  # noqa: E731
+    lins = []
+    for m in (4352, 1024, 4352, 4096):
+        codes = torch.randint(0, 65536, (m, n // 8), generator=g)
+        lins.append((PackedCodes(codes.to(dev), m, n, [0]), sign(m), sign(n), 1.0, 0.0, 0.0135, None))
+    x = torch.randn(B, n, generator=g).to(dev).bfloat16()
+    for lin, y in zip(lins, forward_packed_group(x, lins)):
+        assert torch.equal(y, forward_packed(x, *lin))
