@@ -176,8 +176,9 @@ struct WideMfma {
 // round over the CUs (a partial second round costs more than the split
 // saves: 11008 x 4096 at 512 rows, 172 tiles, runs 3.7 % faster over the
 // step as 1 group than as 2), at most the output kernel's partial-group
-// limit.  Up to 128 rows two work-groups per CU, which run side by side and
-// cover each other's loads, while the partial sums take at most 8 MiB.
+// limit.  Up to 128 rows two work-groups per CU of the decode-in-the-loop
+// kernel, which run side by side and cover each other's loads, while the
+// partial sums take at most 8 MiB and (one stage) no CU gets more slices.
 int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2);
 // Most bytes of partial sums of any wide call of up to B rows, of either stage
 // count (fewer rows can have more groups, and more bytes).

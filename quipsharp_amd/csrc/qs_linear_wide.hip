@@ -572,10 +572,16 @@ static int groups_within(int64_t tiles, int64_t n, int64_t limit) {
 int wide_splits(int64_t m, int64_t n, int64_t B, int ncu, bool has2) {
   const int64_t tiles = wide_tiles(m, n, B, has2);
   int g = groups_within(tiles, n, ncu);
-  // up to 128 rows a second work-group per CU, while the partial sums stay few
+  // up to 128 rows a second work-group per CU, while the partial sums stay few;
+  // with one stage only where no CU then has more slices to go through (8192 x
+  // 5120, 32 rows: five slices each in 4 groups 25.6 us, three and two groups per
+  // CU in 8 29.9; 18944 x 3584: fourteen in one group, five in 3 36.9)
   if (B <= 16 * kWgMaxCols && !use_wp(m, n, B, has2)) {
-    const int g2 = groups_within(tiles, n, 2 * ncu), most = (int)(kWgPartialBytes / (B * m * 4));
-    if (g2 > g && most > g) g = g2 < most ? g2 : most;
+    const int64_t S = n / 256;
+    int64_t g2 = groups_within(tiles, n, 2 * ncu);
+    const int64_t most = kWgPartialBytes / (B * m * 4);
+    if (g2 > most) g2 = most;
+    if (g2 > g && (has2 || (tiles * g2 + ncu - 1) / ncu * ((S + g2 - 1) / g2) <= (S + g - 1) / g)) g = (int)g2;
   }
   return g;
 }
