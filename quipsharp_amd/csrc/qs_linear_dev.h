@@ -127,10 +127,11 @@ int launch_bx_big(const BatchedPass& P, hipStream_t stream);
 int launch_by_big(const BatchedPass* P, int count, hipStream_t stream);
 
 // Transforms of a long batch (qs_linear_rows.hip), one row per wave: the input
-// side from kRowsInMin rows and for every length on the chunk scheme up to 32768,
-// 16384 for fp32 rows (each row and its signs on 16 bytes), the output side from
-// kRowsOutMin rows for lengths beyond the chunk kernels' 12288.
-constexpr int64_t kRowsInMin = 160, kRowsOutMin = 320;
+// side for every length on the chunk scheme up to 32768, 16384 for fp32 rows
+// (each row and its signs on 16 bytes), from kRowsInMin rows, or kRowsInMinLong
+// beyond the chunk kernels' 12288; the output side from kRowsOutMin rows for
+// lengths beyond 12288.
+constexpr int64_t kRowsInMin = 257, kRowsInMinLong = 160, kRowsOutMin = 320;
 bool rows_input_fits(const BatchedPass& P);
 bool rows_output_fits(const BatchedPass& P);
 int launch_wx(const BatchedPass* P, int count, hipStream_t stream);

@@ -32,8 +32,12 @@
 //   input, Qwen3-32B    130 rows 63 -> 53 us, 200 85 -> 57, 512 217 -> 112, 2000 721 -> 282
 //   output beyond 12288 (Llama-3-8B gate + up) 130 rows 29 -> ~46 us, 320 57 -> ~42, 2000 360 -> ~150
 //   output up to 12288 (Llama-2-7B) 512 rows 62 -> 86 us, 2000 201 -> 231: not taken
-// so the input runs here from kRowsInMin rows, the output from kRowsOutMin rows
-// beyond 12288.  The output kernel reads the fp32 partial sums once per group
+//   input, one linear alone (its whole call, 2 bits): 4096 x 4096 160 rows 34.5 -> 36.3, 256 39.6 -> 40.8, 320 39.3
+//     -> 40.7, 512 45.4 -> 44.5; 1024 x 1024 256 rows 20.4 -> 21.9, 320 23.9 -> 23.6; 4096 x 11008 200 rows 51.1 ->
+//     52.5, 256 54.0 -> 52.8; 4096 x 14336 160 rows 55.7 -> 54.6; 4096 to 3 x 4096 200 rows 52.7 -> 53.3, 256 55.0 -> 53.9
+// (up to 256 rows the per-row kernel has every row in work at once), so the
+// input runs here from kRowsInMin rows, beyond 12288 from kRowsInMinLong, and the
+// output from kRowsOutMin rows beyond 12288.  The output kernel reads the fp32 partial sums once per group
 // of 16 slices and splits them each time; up to 12288 qs_linear_batched.hip's
 // by_kernel reads them once.  Groups of a row in one work-group instead of one
 // each (the layer's calls, 2 bits): Qwen2.5-7B 2000 rows 1382 -> 1333 us, 4000
@@ -667,7 +671,8 @@ bool rows_transform_fits(int64_t len, int p) {
 bool rows_input_fits(const BatchedPass& P) {
   const size_t es = P.x_dtype == QS_DTYPE_F32 ? 4 : 2;
   if (P.x_dtype == QS_DTYPE_F32 && P.n > kRowsMaxFp32) return false;
-  return P.frag && P.B >= kRowsInMin && rows_transform_fits(P.n, P.pn) && (reinterpret_cast<uintptr_t>(P.x) & 15) == 0 &&
+  const int64_t rows = chunk_transform_fits(P.n, P.pn) ? kRowsInMin : kRowsInMinLong;
+  return P.frag && P.B >= rows && rows_transform_fits(P.n, P.pn) && (reinterpret_cast<uintptr_t>(P.x) & 15) == 0 &&
          P.ldx * es % 16 == 0 && (reinterpret_cast<uintptr_t>(P.sv) & (P.sbits ? 3 : 15)) == 0;
 }
 bool rows_output_fits(const BatchedPass& P) {

@@ -135,12 +135,12 @@ def structured_T(v):
     return ((a.cos() + a.sin()) / p ** 0.5 @ z).reshape(v.shape)
 
 
-@pytest.mark.parametrize("n", [512, 3584, 11008])
-@pytest.mark.parametrize("B", [159, 160])
+@pytest.mark.parametrize("n,B", [(512, 256), (512, 257), (3584, 256), (3584, 257), (11008, 256), (11008, 257),
+                                 (14336, 160)])
 @pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1.0), (torch.float16, 1.0), (torch.float16, 3e4),
                                         (torch.float32, 1.0)])
 def test_input_factors_that_are_not_signs(dev, n, B, dtype, size):
-    """sv of other values than +-1 on both sides of the threshold: the products
+    """sv of other values than +-1 on both sides of the thresholds: the products
     keep two 16-bit planes, and those beyond fp16's range stay finite."""
     from quipsharp_amd.codebooks.e8p import _decode
     from quipsharp_amd.quantize import forward_packed
