@@ -4,7 +4,7 @@
 // E8P.  At a shift, with magnitudes a_i = |x_i +- 1/4|, a table row with
 // entries T has the distance sum (a_i - T_i)^2, plus 4 min a_i T_i where its
 // signing has the wrong parity (quipsharp/codebooks/e8p.py:104-128, the greedy
-// repair).  Rows 0 .. 226 are every arrangement of nine multisets of entries:
+// repair).  Rows 0 .. 226 are every arrangement of seven multisets of entries:
 // all 1/2 with j = 0 .. 4 entries of 3/2, or with one 5/2 and up to one 3/2
 // (64 rows).  By the rearrangement inequality the best row of a multiset gives
 // the large entries to the large magnitudes, penalty included (the least

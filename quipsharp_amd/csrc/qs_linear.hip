@@ -51,11 +51,12 @@ struct WsLayout {
 };
 
 // From this many activation rows on (more than one 16-row pass), the tiled
-// forward runs the wide GEMM (qs_linear_wide.hip: each code decoded once per
-// up to 256 activation rows, every decoded fragment feeding several MFMAs)
-// instead of decoding the codes once per 16 rows.  Measured at 17..48 rows
-// on the 7B shapes: 24 rows 23 / 34 / 35 us wide against 36 / 47 / 50 us in
-// two 16-row passes (4096x4096, 11008x4096, 4096x11008).
+// forward runs the wide GEMM (qs_linear_wide.hip: a code decoded once or twice
+// per up to 128 activation rows, or once per up to 256, every decoded fragment
+// feeding several MFMAs) instead of decoding the codes once per 16 rows.  One
+// call of 17 rows 19.1 / 28.3 / 29.5 us against 25.7 / 36.5 / 38.3 as 16 + 1, 24
+// rows 19.6 / 30.2 / 29.8 us against 28.8 / 42.5 / 42.9 as 16 + 8 (4096x4096,
+// 11008x4096, 4096x11008, graph-replayed).
 constexpr int64_t kWideMinBatch = 17;
 
 // Work-groups per batch row of the input / output transform: the odd-factor
@@ -674,8 +675,10 @@ using namespace qs;
 // The wide-batch path (tiled codes, kWideMinBatch rows or more): input
 // transform of every row into the fragment-major fp16 operand, the GEMM with
 // the decode in its loop on the matrix cores (qs_linear_wide.hip), output
-// transform of every row.  The chunk-scheme row kernels take the n and m they
-// cover, the LDS-radix kernels the rest.
+// transform of every row.  Long batches are transformed one row per wave
+// (qs_linear_rows.hip); else the chunk-scheme row kernels take the n and m they
+// cover, the kernels of 16 chunks per work-group (qs_linear_big.hip) lengths up to
+// 32768, the LDS-radix kernels the rest.
 static int forward_wide(const void* x, int x_dtype, int64_t ldx, int64_t batch, int64_t n, int64_t m,
                         const void* codes0, const void* codes1, const float* sv, const float* su, int kron_pn,
                         const float* kron_n, int kron_pm, const float* kron_m, float s0, float s1, float layer_scale,
@@ -1083,10 +1086,12 @@ size_t group_prefix_bytes(int count, int64_t n, M m_of) {
 
 // Grouped forward for three or more rows: the input transforms of all the
 // linears in one launch, their decode-matvecs in one launch (16-row pass) or
-// one wide GEMM (kWideMinBatch rows and more; beyond 128 rows of one stage one
-// each, or one for linears of one shape whose tiles fit one round over the CUs), and their
-// output transforms in one launch (a linear whose m is outside the chunk
-// scheme: the whole-row output kernel).  Bit-identical to one
+// one wide GEMM (kWideMinBatch rows and more: one launch for the linears of the
+// decode-in-the-loop kernel; of the producer / consumer kernel up to 128 rows one
+// for those of one m, beyond one each, or one for linears of one shape whose
+// tiles fit one round over the CUs), and their output transforms in one launch
+// for each of the row, chunk and 16-chunk kernels (a linear whose m none of them
+// covers: the whole-row output kernel).  Bit-identical to one
 // qs_linear_forward per linear, except a shared GEMM: its slice groups are the
 // group's, so the outputs equal separate calls up to the fp32 summation order.
 static int forward_group_rows(const void* x, int x_dtype, int64_t ldx, int64_t batch, int64_t n, int kron_pn,

@@ -164,3 +164,10 @@ def test_long_fp32_rows_are_transformed_in_fp32(dev, n):
     args = (packed, su.to(dev), sv.to(dev), 1.0, 0.0, 0.0135)
     x = torch.randn(160, n, generator=torch.Generator().manual_seed(n)).to(dev)
     assert torch.equal(forward_packed(x, *args)[:159], forward_packed(x[:159].contiguous(), *args))
+
+
+@pytest.mark.parametrize("m,n", [(512, 3584), (768, 4096), (256, 11008)])
+@pytest.mark.parametrize("B", [256, 257, 259])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_threshold_up_to_12288_columns(dev, m, n, B, dtype):
+    test_long_batches_match_dense(dev, m, n, B, dtype)
